@@ -191,6 +191,7 @@ static unsigned nbh_create(const nbhip_ctx* ctx, int device, int nsim, const int
         t.body_off = off;
         t.body_n = nbody[k];
         t.first = t.root = t.end = -1;
+        t.odd_mass = 1u;
         if (!(t.eps2 > 0.0)) st->all_eps2_pos = 0;
         st->h_body_off[k] = off;
         st->h_body_n[k] = nbody[k];
@@ -300,6 +301,7 @@ static unsigned nbh_upload_range(nbhip_state* st, int off, int cnt, const double
     }
     NBH_CHECK(hipMemcpyAsync(st->m + off, mass, n * sizeof(double), hipMemcpyHostToDevice,
                              st->stream));
+    nbh_masses_changed(st);
     NBH_CHECK(hipStreamSynchronize(st->stream));
     st->have_tree = 0;
     return NBHIP_SUCCESS;
@@ -600,6 +602,7 @@ extern "C" unsigned nbhip_restore(nbhip_state* st, int sim, unsigned step, doubl
     NBH_CHECK(hipStreamSynchronize(st->stream));
     t.rsize = rsize;
     t.key_scale = 9223372036854775808.0 / rsize;
+    t.odd_mass = 1u;
     NBH_CHECK(hipMemcpyAsync(st->sims + sim, &t, sizeof(t), hipMemcpyHostToDevice, st->stream));
     NBH_CHECK(hipStreamSynchronize(st->stream));
     st->step = step;

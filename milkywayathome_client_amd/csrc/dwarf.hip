@@ -588,6 +588,7 @@ extern "C" unsigned nbhip_mixed_dwarf_state(nbhip_state* st, int sim, const nbhi
     const size_t o = (size_t) st->h_body_off[sim];
     rc = nbh_dwarf_device(p, m, st->px + o, st->py + o, st->pz + o, st->vx + o, st->vy + o,
                           st->vz + o, st->m + o, st->stream);
+    nbh_masses_changed(st);
     if (rc) return rc;
     /* the dark matter is left out of histograms (ignoreBody) */
     std::vector<unsigned char> ig;

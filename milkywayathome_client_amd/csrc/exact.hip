@@ -35,6 +35,7 @@ __device__ __forceinline__ void nbh_exact_range(const SimTab& t, int seg, int& a
 }
 
 /* Forward pair term: nbGravity_Exact's expression order. */
+template <bool PLAIN>
 struct ExactFwd {
     double x0, y0, z0, eps2;
     double ax = 0.0, ay = 0.0, az = 0.0;
@@ -44,18 +45,24 @@ struct ExactFwd {
         const double dy = yk - y0;
         const double dz = zk - z0;
         const double drSq = dz * dz + (dy * dy + dx * dx) + eps2;
-        const double drab = sqrt(drSq);
-        const double phii = mk / drab;
-        const double mor3 = phii / drSq;
+        NbhRoot c;
+        const double mor3 = nbh_mor3<PLAIN>(mk, drSq, c);
         ax += mor3 * dx;
         ay += mor3 * dy;
         az += mor3 * dz;
+    }
+    __device__ __forceinline__ void store(double* p, size_t N) const
+    {
+        p[0] = ax;
+        p[N] = ay;
+        p[2 * N] = az;
     }
 };
 
 /* Adjoint pair term: (J^T g)_i = sum_k T(d_ik) (m_i g_k - m_k g_i),
  * dL/dm_i = -sum_k g_k . d_ik / s^3, d_ik = x_k - x_i,
  * T(d) = I / s^3 - 3 d d^T / s^5 (the self term vanishes identically). */
+template <bool PLAIN>
 struct ExactAdj {
     double x0, y0, z0, eps2, mi, gi0, gi1, gi2;
     double ox = 0.0, oy = 0.0, oz = 0.0, om = 0.0;
@@ -64,8 +71,16 @@ struct ExactAdj {
     {
         const double dx = xk - x0, dy = yk - y0, dz = zk - z0;
         const double s2 = dx * dx + dy * dy + dz * dz + eps2;
-        const double s3 = 1.0 / (s2 * sqrt(s2));
-        const double s5 = s3 / s2;
+        double s3, s5;
+        if (PLAIN) {
+            const NbhRoot c = nbh_root(s2);
+            const double d3 = s2 * c.r;
+            s3 = nbh_recip_refine(d3, nbh_recip_refine(d3, c.ir2 * c.ir));
+            s5 = nbh_quot(s3, s2, c.ir2);
+        } else {
+            s3 = 1.0 / (s2 * sqrt(s2));
+            s5 = s3 / s2;
+        }
         const double w0 = mi * gk0 - mk * gi0;
         const double w1 = mi * gk1 - mk * gi1;
         const double w2 = mi * gk2 - mk * gi2;
@@ -74,6 +89,13 @@ struct ExactAdj {
         oy += s3 * w1 - 3.0 * s5 * dw * dy;
         oz += s3 * w2 - 3.0 * s5 * dw * dz;
         om -= (gk0 * dx + gk1 * dy + gk2 * dz) * s3;
+    }
+    __device__ __forceinline__ void store(double* p, size_t N) const
+    {
+        p[0] = ox;
+        p[N] = oy;
+        p[2 * N] = oz;
+        p[3 * N] = om;
     }
 };
 
@@ -114,62 +136,63 @@ __global__ __launch_bounds__(256) void k_exact_part(int n, const double* __restr
         eps2 = t.eps2;
     }
     const double x0 = valid ? px[i] : 0.0, y0 = valid ? py[i] : 0.0, z0 = valid ? pz[i] : 0.0;
-    ExactFwd F;
-    ExactAdj G;
-    if (ADJ) {
-        G.x0 = x0; G.y0 = y0; G.z0 = z0; G.eps2 = eps2;
-        G.mi = valid ? m[i] : 0.0;
-        G.gi0 = valid ? ga[i] : 0.0;
-        G.gi1 = valid ? ga[N + i] : 0.0;
-        G.gi2 = valid ? ga[2 * N + i] : 0.0;
-    } else {
-        F.x0 = x0; F.y0 = y0; F.z0 = z0; F.eps2 = eps2;
-    }
-
-    if (uniform) {
-        /* every body of the workgroup sums the same segment */
-        int ua, ub;
-        nbh_exact_range(sims[sim0], seg, ua, ub);
-        if (ua >= ub) return;                     /* whole workgroup: no barrier follows */
-        for (int base = ua; base < ub; base += NBH_EXACT_TILE) {
-            const int k = base + tid;
-            if (k < ub) {
-                tile[tid] = make_double4(px[k], py[k], pz[k], m[k]);
-                if (ADJ) tileg[tid] = make_double4(ga[k], ga[N + k], ga[2 * N + k], 0.0);
-            }
-            __syncthreads();
-            const int cnt = min(NBH_EXACT_TILE, ub - base);
-            for (int j = 0; j < cnt; ++j) {
-                const double4 s = tile[j];
-                if (ADJ) {
-                    const double4 gk = tileg[j];
-                    G.add(s.x, s.y, s.z, s.w, gk.x, gk.y, gk.z);
-                } else {
-                    F.add(s.x, s.y, s.z, s.w);
+    /* the segment through one pair functor (add: 4 or 7 source values) */
+    auto sum = [&](auto& P) {
+        if (uniform) {
+            /* every body of the workgroup sums the same segment */
+            int ua, ub;
+            nbh_exact_range(sims[sim0], seg, ua, ub);
+            for (int base = ua; base < ub; base += NBH_EXACT_TILE) {
+                const int k = base + tid;
+                if (k < ub) {
+                    tile[tid] = make_double4(px[k], py[k], pz[k], m[k]);
+                    if constexpr (ADJ)
+                        tileg[tid] = make_double4(ga[k], ga[N + k], ga[2 * N + k], 0.0);
                 }
+                __syncthreads();
+                const int cnt = min(NBH_EXACT_TILE, ub - base);
+                #pragma unroll 2
+                for (int j = 0; j < cnt; ++j) {
+                    const double4 s = tile[j];
+                    if constexpr (ADJ) {
+                        const double4 gk = tileg[j];
+                        P.add(s.x, s.y, s.z, s.w, gk.x, gk.y, gk.z);
+                    } else {
+                        P.add(s.x, s.y, s.z, s.w);
+                    }
+                }
+                __syncthreads();
             }
-            __syncthreads();
+        } else {
+            for (int k = a; k < b; ++k) {
+                if constexpr (ADJ)
+                    P.add(px[k], py[k], pz[k], m[k], ga[k], ga[N + k], ga[2 * N + k]);
+                else
+                    P.add(px[k], py[k], pz[k], m[k]);
+            }
         }
-    } else {
-        for (int k = a; k < b; ++k) {
-            if (ADJ)
-                G.add(px[k], py[k], pz[k], m[k], ga[k], ga[N + k], ga[2 * N + k]);
-            else
-                F.add(px[k], py[k], pz[k], m[k]);
+        if (!valid || a >= b) return;
+        constexpr int W = ADJ ? 4 : 3;
+        double* p = part + (size_t) seg * W * N + i;
+        P.store(p, N);
+    };
+    auto run = [&](auto P) {
+        P.x0 = x0; P.y0 = y0; P.z0 = z0; P.eps2 = eps2;
+        if constexpr (ADJ) {
+            P.mi = valid ? m[i] : 0.0;
+            P.gi0 = valid ? ga[i] : 0.0;
+            P.gi1 = valid ? ga[N + i] : 0.0;
+            P.gi2 = valid ? ga[2 * N + i] : 0.0;
         }
-    }
-    if (!valid || a >= b) return;
-    constexpr int W = ADJ ? 4 : 3;
-    double* p = part + (size_t) seg * W * N + i;
-    if (ADJ) {
-        p[0] = G.ox;
-        p[N] = G.oy;
-        p[2 * N] = G.oz;
-        p[3 * N] = G.om;
+        sum(P);
+    };
+    /* one simulation: the whole workgroup goes one way, barriers included */
+    const bool plain = uniform ? nbh_plain_range(sims[sim0])
+                               : (valid && nbh_plain_range(sims[sim]));
+    if constexpr (ADJ) {
+        if (plain) run(ExactAdj<true>()); else run(ExactAdj<false>());
     } else {
-        p[0] = F.ax;
-        p[N] = F.ay;
-        p[2 * N] = F.az;
+        if (plain) run(ExactFwd<true>()); else run(ExactFwd<false>());
     }
 }
 

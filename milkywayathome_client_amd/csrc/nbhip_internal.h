@@ -75,6 +75,9 @@ struct SimTab {
     int maxdepth;
     unsigned flags;                /* sticky NBHIP_* bits of this simulation */
     unsigned incest;               /* a body of this simulation missed itself */
+    unsigned odd_mass;             /* a mass was nonzero and outside the range of the unscaled
+                                      divisions (nbh_plain_range), or none was looked at yet */
+    unsigned odd_seen;             /* the same, gathered by the bbox pass that is running */
 };
 
 /* Device-resident scalars shared by all simulations of a state. */
@@ -264,6 +267,7 @@ void nbh_bbox(nbhip_state* st, int drift);
 void nbh_build(nbhip_state* st, int graph_safe);
 unsigned nbh_level_lists(nbhip_state* st);
 void nbh_step_end(nbhip_state* st);
+void nbh_masses_changed(nbhip_state* st);
 /* launchers (walk.hip) */
 void nbh_walk(nbhip_state* st, int kick, int count, double* out_ax, double* out_ay,
               double* out_az, int self_only, const WalkTune* tune);

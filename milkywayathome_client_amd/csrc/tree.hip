@@ -77,8 +77,11 @@ __global__ __launch_bounds__(256) void k_drift_bbox(int n, int drift, double dt,
             vx[i] = ux; vy[i] = uy; vz[i] = uz;
             px[i] = x; py[i] = y; pz[i] = z;
         }
-        pos4[i] = make_double4(x, y, z, m[i]);     /* gathered by the tree build */
+        const double mi = m[i];
+        pos4[i] = make_double4(x, y, z, mi);       /* gathered by the tree build */
         const int sim = simid[i];
+        if (mi != 0.0 && !(mi >= NBH_PLAIN_MASS_MIN && mi <= NBH_PLAIN_MASS_MAX))
+            sims[sim].odd_seen = 1u;               /* every writer stores 1 */
         if (sim != cur) {
             if (cur >= 0) nbh_max_bits(sims, cur, mx);
             cur = sim;
@@ -137,6 +140,8 @@ __global__ __launch_bounds__(256) void k_rsize(int nsim, SimTab* __restrict__ si
         } else {
             while (r < 2.0 * xm) r *= 2.0;
         }
+        t.odd_mass = t.odd_seen;
+        t.odd_seen = 0u;
         t.rsize = r;
         t.key_scale = 9223372036854775808.0 / r;
         t.xyzmax_bits = 0ull;
@@ -1817,6 +1822,19 @@ void nbh_bbox(nbhip_state* st, int drift)
                        st->n, drift, dt, 0.5 * dt, st->px, st->py, st->pz, st->vx, st->vy, st->vz,
                        st->ax, st->ay, st->az, st->m, st->pos4, st->simid, st->sims, st->scal);
     hipLaunchKernelGGL(k_rsize, dim3(1), dim3(256), 0, st->stream, st->nsim, st->sims, st->scal);
+}
+
+/* New masses: no pass has looked at them yet (nbh_plain_range). */
+__global__ __launch_bounds__(256) void k_masses_changed(int nsim, SimTab* __restrict__ sims)
+{
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < nsim; k += gridDim.x * 256)
+        sims[k].odd_mass = 1u;
+}
+
+void nbh_masses_changed(nbhip_state* st)
+{
+    hipLaunchKernelGGL(k_masses_changed, dim3(nbh_blocks(st->nsim, 256)), dim3(256), 0,
+                       st->stream, st->nsim, st->sims);
 }
 
 void nbh_step_end(nbhip_state* st)

@@ -19,6 +19,37 @@ struct Quad6 {
     double q[6];
 };
 
+/* One accepted node added to a body's acceleration: the reference's
+ * expressions in its operation order (nbGravity, nbody/src/nbody_grav.c:
+ * 53-99); r2 is the softened squared distance. */
+template <bool QUAD, bool PLAIN>
+__device__ __forceinline__ void nbh_interact64(double r2, double m, bool cell, const Quad6& nq,
+                                               double dx, double dy, double dz, double& ax,
+                                               double& ay, double& az)
+{
+    NbhRoot c;
+    const double mor3 = nbh_mor3<PLAIN>(m, r2, c);
+    ax += mor3 * dx;
+    ay += mor3 * dy;
+    az += mor3 * dz;
+    if (QUAD && cell) {
+        const double qxx = nq.q[0], qxy = nq.q[1], qxz = nq.q[2];
+        const double qyy = nq.q[3], qyz = nq.q[4], qzz = nq.q[5];
+        const double qx = qxx * dx + qxy * dy + qxz * dz;
+        const double qy = qxy * dx + qyy * dy + qyz * dz;
+        const double qz = qxz * dx + qyz * dy + qzz * dz;
+        const double drQdr = qx * dx + qy * dy + qz * dz;
+        const double dr5inv = nbh_dr5<PLAIN>(r2, c);
+        const double phiQ = nbh_phiq<PLAIN>(dr5inv, drQdr, r2, c);
+        ax += phiQ * dx;
+        ay += phiQ * dy;
+        az += phiQ * dz;
+        ax -= dr5inv * qx;
+        ay -= dr5inv * qy;
+        az -= dr5inv * qz;
+    }
+}
+
 /* Plain form: FP64 end to end, reference operation order. */
 template <int BS, bool QUAD, bool COUNT>
 __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
@@ -46,6 +77,9 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
     int lp = L.lp;
     const double eps2 = L.eps2;
     const bool eps2_pos = o.all_eps2_pos;
+    /* every simulation of the wave clear of the exponent range's ends */
+    const bool plain =
+        __builtin_amdgcn_ballot_w64(valid && !nbh_plain_range(sims[L.sim])) == 0ull;
     double ax = 0.0, ay = 0.0, az = 0.0;
     bool met = false;
     unsigned nbb = 0, nbc = 0, nop = 0, steps = 0;
@@ -67,7 +101,7 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
         const double dx = nd.x - p.x;
         const double dy = nd.y - p.y;
         const double dz = nd.z - p.z;
-        double drSq = dz * dz + (dy * dy + dx * dx);
+        const double drSq = dz * dz + (dy * dy + dx * dx);
         const bool accept = active && (nd_body >= 0 || drSq >= nd.rcrit2);
         const bool open = active && !accept;
         const bool any_open = __builtin_amdgcn_ballot_w64(open) != 0ull;
@@ -83,29 +117,12 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
             /* with eps2 > 0 the self term adds exactly +0 (dx = dy = dz = 0),
              * so lanes need not branch around it */
             if (eps2_pos || nd_body != self) {
-                drSq += eps2;
-                const double drab = sqrt(drSq);
-                const double phii = nd.m / drab;
-                const double mor3 = phii / drSq;
-                ax += mor3 * dx;
-                ay += mor3 * dy;
-                az += mor3 * dz;
-                if (QUAD && nd_body < 0) {
-                    const double qxx = nq.q[0], qxy = nq.q[1], qxz = nq.q[2];
-                    const double qyy = nq.q[3], qyz = nq.q[4], qzz = nq.q[5];
-                    const double qx = qxx * dx + qxy * dy + qxz * dz;
-                    const double qy = qxy * dx + qyy * dy + qyz * dz;
-                    const double qz = qxz * dx + qyz * dy + qzz * dz;
-                    const double drQdr = qx * dx + qy * dy + qz * dz;
-                    const double dr5inv = 1.0 / ((drSq * drSq) * drab);
-                    const double phiQ = 2.5 * (dr5inv * drQdr) / drSq;
-                    ax += phiQ * dx;
-                    ay += phiQ * dy;
-                    az += phiQ * dz;
-                    ax -= dr5inv * qx;
-                    ay -= dr5inv * qy;
-                    az -= dr5inv * qz;
-                }
+                if (plain)
+                    nbh_interact64<QUAD, true>(drSq + eps2, nd.m, nd_body < 0, nq, dx, dy, dz, ax,
+                                               ay, az);
+                else
+                    nbh_interact64<QUAD, false>(drSq + eps2, nd.m, nd_body < 0, nq, dx, dy, dz,
+                                                ax, ay, az);
                 if (COUNT) {
                     if (nd_body >= 0) nbb += nd_body != self; else ++nbc;
                 }
