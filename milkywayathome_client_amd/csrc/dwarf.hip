@@ -132,38 +132,55 @@ __host__ __device__ inline double nbh_psi_total(const Model& m, double r)
 
 /* f_c(E) by Eddington's formula: 2 int_0^sqrt(E) g(E - t^2) dt / (sqrt(8) pi^2)
  * with g = d^2 rho_c / d psi^2 at the radius where the total psi equals
- * E - t^2 (found by bisection in ln r). */
-__global__ void k_df_table(Model m, int comp, const double* __restrict__ gx,
-                           const double* __restrict__ gw, double* __restrict__ lnf)
+ * E - t^2 (found by bisection in ln r).
+ *
+ * One workgroup per energy, one thread per quadrature node: the bisection (80
+ * dependent steps of an exp and two potentials) is the whole cost, so it is
+ * spread over 2048 x 128 threads and shared by both components, whose
+ * integrands sit at the same radii.  The 128 terms are then added in node
+ * order by one lane per component, as a single thread would (the same bits).
+ * With one thread per energy and component walking its 128 nodes (64 waves in
+ * all) the two tables took 2 x 6.9 ms. */
+__global__ __launch_bounds__(kGauss) void k_df_table(Model m, const double* __restrict__ gx,
+                                                     const double* __restrict__ gw,
+                                                     double* __restrict__ lnf)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= kTable) return;
+    __shared__ double term[2][kGauss];
+    const int k = blockIdx.x;
+    const int j = threadIdx.x;
     const double E = exp(m.lnE0 + m.dlnE * k);
     const double se = sqrt(E);
     const double amin = fmin(m.c[0].a, m.c[1].a), amax = fmax(m.c[0].a, m.c[1].a);
-    double acc = 0.0;
-    for (int j = 0; j < kGauss; ++j) {
-        const double t = 0.5 * se * (gx[j] + 1.0);
-        const double psi = E - t * t;
-        /* ln r with psi_total(r) = psi (psi decreases with r) */
-        double lo = log(amin) - 30.0, hi = log(amax) + 40.0;
-        for (int it = 0; it < 80; ++it) {
-            const double mid = 0.5 * (lo + hi);
-            if (nbh_psi_total(m, exp(mid)) > psi) lo = mid; else hi = mid;
-        }
-        const double r = exp(0.5 * (lo + hi));
-        double rf, r1, r2, p0, p1, p2, q0, q1, q2;
-        nbh_rho(m.c[comp], r, &rf, &r1, &r2);
-        nbh_psi(m.c[0], r, &p0, &p1, &p2);
-        nbh_psi(m.c[1], r, &q0, &q1, &q2);
-        const double d1 = p1 + q1, d2 = p2 + q2;
-        const double g = (r2 * d1 - r1 * d2) / (d1 * d1 * d1);
-        acc += gw[j] * g;
+    const double t = 0.5 * se * (gx[j] + 1.0);
+    const double psi = E - t * t;
+    /* ln r with psi_total(r) = psi (psi decreases with r) */
+    double lo = log(amin) - 30.0, hi = log(amax) + 40.0;
+    for (int it = 0; it < 80; ++it) {
+        const double mid = 0.5 * (lo + hi);
+        if (nbh_psi_total(m, exp(mid)) > psi) lo = mid; else hi = mid;
     }
+    const double r = exp(0.5 * (lo + hi));
+    double p0, p1, p2, q0, q1, q2;
+    nbh_psi(m.c[0], r, &p0, &p1, &p2);
+    nbh_psi(m.c[1], r, &q0, &q1, &q2);
+    const double d1 = p1 + q1, d2 = p2 + q2;
+    for (int comp = 0; comp < 2; ++comp) {
+        double rf, r1, r2;
+        nbh_rho(m.c[comp], r, &rf, &r1, &r2);
+        const double g = (r2 * d1 - r1 * d2) / (d1 * d1 * d1);
+        term[comp][j] = gw[j] * g;
+    }
+    __syncthreads();
+    if (j & 63) return;
+    const int comp = j >> 6;
+    double acc = 0.0;
+    #pragma unroll 8
+    for (int i = 0; i < kGauss; ++i) acc += term[comp][i];
     /* 2 * (se / 2) * sum = se * sum */
     const double f = se * acc / (sqrt(8.0) * M_PI * M_PI);
-    lnf[k] = f > 0.0 ? log(f) : -INFINITY;
+    lnf[comp * kTable + k] = f > 0.0 ? log(f) : -INFINITY;
 }
+static_assert(kGauss == 128, "k_df_table: one wave's first lane per component");
 
 __device__ inline double nbh_df(const Model& m, const double* __restrict__ lnf, double E)
 {
@@ -218,6 +235,65 @@ __device__ inline bool nbh_direction(Stream& s, double* u)
     return false;
 }
 
+/* The radius of body i (one lane per body, every lane of the wave here):
+ * r_mag's rejection, trial t drawing block t of the body's stream.  A Plummer
+ * sphere accepts one trial in 140 (it is cut at 50 scale radii), so a wave
+ * whose lanes each try for themselves runs until its unluckiest body, some
+ * 660 rounds.  The trials of a body are independent, so the lanes are dealt
+ * out anew each round over the bodies still without a radius, 64 / pending
+ * consecutive trials each, and a body takes its first accepted one: the same
+ * trial, in about 190 rounds (the sampler kernel: 1.1 -> 0.43 ms at 200 000
+ * bodies).  trials: blocks drawn; false past kMaxTries. */
+__device__ inline bool nbh_radius(const Model& m, unsigned i, double& r, unsigned& trials)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned base = i - (unsigned) lane;
+    const unsigned key[2] = { (unsigned) m.seed, (unsigned) (m.seed >> 32) };
+    unsigned next = 0;                             /* this lane's body: its next trial */
+    bool ok = false;
+    unsigned long long pend = __ballot(i < m.nbody);
+    while (pend) {
+        const int np = __popcll(pend);
+        const int per = 64 / np;
+        /* the slot-th pending body takes lanes [slot * per, (slot + 1) * per) */
+        const int rank = __popcll(pend & ((1ull << lane) - 1ull));
+        const bool mine = (pend >> lane) & 1ull;
+        const int slot = lane / per, sub = lane - slot * per;
+        /* pending lanes sorted to the front: sorted[k] = the k-th of them */
+        const int sorted = __builtin_amdgcn_ds_permute((mine ? rank : np + lane - rank) * 4, lane);
+        const int owner = __shfl(sorted, slot < np ? slot : 0, 64);
+        const unsigned t = (unsigned) __shfl((int) next, owner, 64) + (unsigned) sub;
+        const unsigned body = base + (unsigned) owner;
+        const int comp = body < m.nbody_baryon ? 0 : 1;
+        double x = 0.0;
+        bool hit = false;
+        if (slot < np && t < (unsigned) kMaxTries) {
+            const unsigned ctr[4] = { body, t, 0u, 0x64776172u };
+            unsigned o[4];
+            nbh_philox4x32_10(ctr, key, o);
+            x = nbh_u01(o[0], o[1]) * m.bound[comp];
+            const double u = nbh_u01(o[2], o[3]);
+            double f, d1, d2;
+            nbh_rho(m.c[comp], x, &f, &d1, &d2);
+            hit = x > 0.0 && x * x * f / m.r2rho_max[comp] > u;
+        }
+        const unsigned long long hits = __ballot(hit);
+        const unsigned long long own =
+            mine ? (hits >> (rank * per)) & (per == 64 ? ~0ull : (1ull << per) - 1ull) : 0ull;
+        const int first = own ? __builtin_ctzll(own) : 0;
+        const double xv = __shfl(x, mine ? rank * per + first : lane, 64);
+        if (own) {
+            r = xv;
+            trials = next + (unsigned) first + 1u;
+            ok = true;
+        } else if (mine) {
+            next += (unsigned) per;
+        }
+        pend = __ballot(mine && !own && next < (unsigned) kMaxTries);
+    }
+    return ok;
+}
+
 __global__ __launch_bounds__(256) void k_dwarf_sample(Model m, const double* __restrict__ lnf,
                                                       double* __restrict__ px,
                                                       double* __restrict__ py,
@@ -229,26 +305,18 @@ __global__ __launch_bounds__(256) void k_dwarf_sample(Model m, const double* __r
                                                       unsigned* __restrict__ fail)
 {
     const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    unsigned trials = 0;
+    double r = 0.0;
+    bool ok = nbh_radius(m, i, r, trials);
     if (i >= m.nbody) return;
     const int comp = i < m.nbody_baryon ? 0 : 1;
-    const Comp c = m.c[comp];
     const double* tab = lnf + (size_t) comp * kTable;
     Stream s;
     s.key[0] = (unsigned) m.seed;
     s.key[1] = (unsigned) (m.seed >> 32);
     s.body = i;
-    s.n = 0;
+    s.n = trials;                      /* a radius trial is one block of two draws */
     s.left = 0;
-    bool ok = false;
-    /* radius: r_mag's rejection */
-    double r = 0.0;
-    for (int t = 0; t < kMaxTries && !ok; ++t) {
-        r = s.next() * m.bound[comp];
-        const double u = s.next();
-        double f, d1, d2;
-        nbh_rho(c, r, &f, &d1, &d2);
-        ok = r > 0.0 && r * r * f / m.r2rho_max[comp] > u;
-    }
     /* speed: rejection against v^2 f(psi(r) - v^2 / 2) below 0.99 v_esc,
      * under an envelope from a scan of the speeds */
     const double psi = nbh_psi_total(m, r);
@@ -326,6 +394,7 @@ __global__ void k_dwarf_total(int nblocks, const double* __restrict__ part,
     const int q = threadIdx.x;
     if (q >= 12) return;
     double s = 0.0;
+    #pragma unroll 16                  /* the loads of 16 blocks in flight, added in order */
     for (int b = 0; b < nblocks; ++b) s += part[12 * (size_t) b + q];
     const double mass = q < 6 ? m_light : m_dark;
     cm[q] = mass > 0.0 ? s / mass : 0.0;
@@ -444,9 +513,8 @@ unsigned nbh_tables(const Model& m, double* d_lnf, double* d_gauss, hipStream_t 
     nbh_gauss_legendre(kGauss, g.data(), g.data() + kGauss);
     NBH_CHECK(hipMemcpyAsync(d_gauss, g.data(), g.size() * sizeof(double), hipMemcpyHostToDevice,
                              s));
-    for (int comp = 0; comp < 2; ++comp)
-        hipLaunchKernelGGL(k_df_table, dim3((kTable + 127) / 128), dim3(128), 0, s, m, comp,
-                           d_gauss, d_gauss + kGauss, d_lnf + comp * kTable);
+    hipLaunchKernelGGL(k_df_table, dim3(kTable), dim3(kGauss), 0, s, m, d_gauss, d_gauss + kGauss,
+                       d_lnf);
     NBH_CHECK(hipGetLastError());
     return NBHIP_SUCCESS;
 }
