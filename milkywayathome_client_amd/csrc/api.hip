@@ -1249,20 +1249,12 @@ extern "C" unsigned nbhip_histogram_dispersion(nbhip_state* st, int sim,
         return NBHIP_SUCCESS;
     }
     const size_t nblk = ((size_t) cnt + 1023) / 1024;
-    /* one scratch block, kept by the state and grown on demand: body bins,
-     * five values per body, per-workgroup partial sums, per-bin state and
-     * the 14 output rows, each section 256-byte aligned */
-    auto up = [](size_t bytes) { return (bytes + 255) & ~(size_t) 255; };
-    const size_t o_val = up((size_t) cnt * sizeof(int));
-    const size_t o_part = o_val + up(5 * (size_t) cnt * sizeof(double));
-    const size_t n_part = 16 * nblk * nbin;
-    if (n_part > ((size_t) 1 << 31)) {
+    if (16 * nblk * nbin > ((size_t) 1 << 31)) {
         nbh_set_error("nbhip_histogram_dispersion: %zu bins x %d bodies is too large", nbin, cnt);
         return NBHIP_USER_ERROR;
     }
-    const size_t o_state = o_part + up(n_part * sizeof(double));
-    const size_t o_out = o_state + up(32 * nbin * sizeof(double));
-    const size_t need = o_out + up(14 * nbin * sizeof(double));
+    /* one scratch block, kept by the state and grown on demand */
+    const size_t need = nbh_disp_bytes(cnt, nbin);
     hipError_t e = hipSuccess;
     if (need > st->disp_cap) {
         if (st->disp_buf) e = hipFree(st->disp_buf);
@@ -1272,11 +1264,7 @@ extern "C" unsigned nbhip_histogram_dispersion(nbhip_state* st, int sim,
         if (e == hipSuccess) st->disp_cap = need;
     }
     if (e == hipSuccess) {
-        char* b = st->disp_buf;
-        double* dout = reinterpret_cast<double*>(b + o_out);
-        nbh_dispersion(st, off, cnt, hp, dp, reinterpret_cast<int*>(b),
-                       reinterpret_cast<double*>(b + o_val), reinterpret_cast<double*>(b + o_part),
-                       reinterpret_cast<double*>(b + o_state), dout);
+        const double* dout = nbh_dispersion(st, off, cnt, hp, dp, st->disp_buf);
         e = hipGetLastError();
         if (e == hipSuccess)
             e = hipMemcpyAsync(out, dout, 14 * nbin * sizeof(double), hipMemcpyDeviceToHost,

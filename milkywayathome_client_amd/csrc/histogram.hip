@@ -52,46 +52,50 @@ __global__ __launch_bounds__(256) void k_histogram(int n, const double* __restri
                                                    const double* __restrict__ pz,
                                                    const unsigned char* __restrict__ ignore,
                                                    const int* __restrict__ simid, HistParams h,
-                                                   unsigned* __restrict__ counts,
+                                                   int per, unsigned* __restrict__ counts,
                                                    unsigned* __restrict__ totals)
 {
     __shared__ unsigned lds[NBH_HIST_LDS];
     __shared__ int s_sim;
     __shared__ int s_mixed;
     const int nbin = h.lbins * h.bbins;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const bool valid = i < n;
-    const int sim = valid ? simid[i] : -1;
+    /* per bodies a thread, 256 apart: bodies [base, base + 256 per) */
+    const int base = blockIdx.x * 256 * per;
+    const int hi = min(n, base + 256 * per);
     if (threadIdx.x == 0) {
-        s_sim = simid[blockIdx.x * 256];
+        s_sim = simid[base];
         s_mixed = 0;
     }
     for (int k = threadIdx.x; k < nbin && k < NBH_HIST_LDS; k += 256) lds[k] = 0u;
     __syncthreads();
-    if (valid && sim != s_sim) s_mixed = 1;       /* benign race: any writer sets 1 */
+    for (int i = base + (int) threadIdx.x; i < hi; i += 256)
+        if (simid[i] != s_sim) s_mixed = 1;       /* benign race: any writer sets 1 */
     __syncthreads();
     const bool local = !s_mixed && nbin <= NBH_HIST_LDS;
 
-    int bin = -1;
-    if (valid && !(ignore && ignore[i])) {
+    for (int i = base + (int) threadIdx.x; i < hi; i += 256) {
+        if (ignore && ignore[i]) continue;
         double beta;
-        bin = nbh_lambda_beta_bin(h, px[i], py[i], pz[i], beta);
-    }
-    if (local) {
-        if (bin >= 0) atomicAdd(&lds[bin], 1u);
-        __syncthreads();
-        unsigned tot = 0;
-        for (int k = threadIdx.x; k < nbin; k += 256) {
-            const unsigned c = lds[k];
-            if (c) atomicAdd(&counts[(size_t) s_sim * nbin + k], c);
-            tot += c;
+        const int bin = nbh_lambda_beta_bin(h, px[i], py[i], pz[i], beta);
+        if (bin < 0) continue;
+        if (local) {
+            atomicAdd(&lds[bin], 1u);
+        } else {
+            const int sim = simid[i];
+            atomicAdd(&counts[(size_t) sim * nbin + bin], 1u);
+            atomicAdd(&totals[sim], 1u);
         }
-        tot = nbh_wave_sum_u32(tot);
-        if (__lane_id() == 0 && tot) atomicAdd(&totals[s_sim], tot);
-    } else if (bin >= 0) {
-        atomicAdd(&counts[(size_t) sim * nbin + bin], 1u);
-        atomicAdd(&totals[sim], 1u);
     }
+    if (!local) return;
+    __syncthreads();
+    unsigned tot = 0;
+    for (int k = threadIdx.x; k < nbin; k += 256) {
+        const unsigned c = lds[k];
+        if (c) atomicAdd(&counts[(size_t) s_sim * nbin + k], c);
+        tot += c;
+    }
+    tot = nbh_wave_sum_u32(tot);
+    if (__lane_id() == 0 && tot) atomicAdd(&totals[s_sim], tot);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -108,15 +112,23 @@ __global__ __launch_bounds__(256) void k_histogram(int n, const double* __restri
  * sigma and correction; so do 4 and 1), so five quantities suffice: q = 0
  * beta, 1 v_los, 2 distance, 3 mu_dec, 4 mu_ra.
  *
- * k_disp_values records each body's bin (-1: ignored or outside) and the
- * three values once.  Each round of sums is k_disp_part, one workgroup per
- * 1024 consecutive bodies with a thread per bin that adds the workgroup's
- * bodies in body order, then k_disp_finish, a thread per bin that adds the
- * workgroups' partial sums in workgroup order and applies nbCalcDisp.  The
+ * k_disp_values takes 1024 consecutive bodies a workgroup (a tile), evaluates
+ * each body's bin and five values once, and stores the tile's binned bodies
+ * sorted by bin, body order kept inside a bin, with the bins' runs.  Each
+ * round of sums is k_disp_part, a thread per (run, quantity) that adds its
+ * run's bodies in body order, then k_disp_finish, a workgroup per bin that
+ * adds the tiles' partial sums in tile order and applies nbCalcDisp.  The
  * sums are therefore deterministic (independent of timing and batching) and
  * differ from the reference's single running sum only in association.
  * Round 0 takes every binned body; each later round keeps a body when
- * |mean - value| < sigma * dispersion of the previous round. */
+ * |mean - value| < sigma * dispersion of the previous round.
+ *
+ * What bounds it: short dependent chains.  Before the bodies were sorted, a
+ * thread per bin looked at all 1024 bodies of its tile (50 of 256 threads
+ * busy, 309 us a round at 10^6 bodies and 50 bins), and a thread per bin then
+ * read 977 tiles' sums one after another (447 us a round); now they take 17
+ * and 24 us, the tiles' sums arriving 32 at a time while the last 32 are
+ * added. */
 #define NBH_DISP_TILE 1024
 #define NBH_DISP_Q 5
 #define NBH_DISP_W (3 * NBH_DISP_Q + 1)   /* per q: sum, sq, removed; then count */
@@ -168,6 +180,15 @@ __device__ __forceinline__ void nbh_proper_motion(const PMFrame& f, double sun, 
     mura = (cra / dist) * 180.0 / M_PI * 3600.0 / 1000000.0;
 }
 
+/* Tile records of k_disp_values: sorted values (q-major inside the tile), the
+ * runs' first positions (nrun + 1 of them) and bins, and the run count. */
+struct DispTile {
+    double* val;         /* [tile][NBH_DISP_Q][NBH_DISP_TILE] */
+    int* start;          /* [tile][NBH_DISP_TILE + 1] */
+    int* bin;            /* [tile][NBH_DISP_TILE] */
+    int* nrun;           /* [tile] */
+};
+
 __global__ __launch_bounds__(256) void k_disp_values(int off, int cnt,
                                                      const double* __restrict__ px,
                                                      const double* __restrict__ py,
@@ -176,72 +197,134 @@ __global__ __launch_bounds__(256) void k_disp_values(int off, int cnt,
                                                      const double* __restrict__ vy,
                                                      const double* __restrict__ vz,
                                                      const unsigned char* __restrict__ ignore,
-                                                     HistParams h, PMFrame f,
-                                                     int* __restrict__ dbin,
-                                                     double* __restrict__ dval)
+                                                     HistParams h, PMFrame f, DispTile T)
 {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= cnt) return;
-    const int i = off + k;
-    int bin = -1;
-    double beta = 0.0, vl = 0.0, dist = 0.0, mudec = 0.0, mura = 0.0;
-    if (!(ignore && ignore[i])) {
-        const double x = px[i], y = py[i], z = pz[i];
-        bin = nbh_lambda_beta_bin(h, x, y, z, beta);
-        const double xs = x + h.sun;
-        const double mag = sqrt(xs * xs + y * y + z * z);
-        vl = (xs * vx[i] + y * vy[i] + z * vz[i]) / mag;
-        dist = mag;
-        nbh_proper_motion(f, h.sun, x, y, z, vx[i], vy[i], vz[i], mudec, mura);
-    }
-    dbin[k] = bin;
-    dval[k] = beta;
-    dval[(size_t) cnt + k] = vl;
-    dval[2 * (size_t) cnt + k] = dist;
-    dval[3 * (size_t) cnt + k] = mudec;
-    dval[4 * (size_t) cnt + k] = mura;
-}
-
-__global__ __launch_bounds__(256) void k_disp_part(int cnt, int nbin, int initial, DispRound r,
-                                                   const int* __restrict__ dbin,
-                                                   const double* __restrict__ dval,
-                                                   const double* __restrict__ state,
-                                                   double* __restrict__ part)
-{
-    __shared__ int sb[NBH_DISP_TILE];
+    /* sort keys: bin, then the body's place in the tile (a stable order);
+     * bodies outside the histogram sort last */
+    __shared__ unsigned long long key[NBH_DISP_TILE];
     __shared__ double sv[NBH_DISP_Q][NBH_DISP_TILE];
+    __shared__ int wsum[4];
+    const int tid = threadIdx.x;
     const int base = blockIdx.x * NBH_DISP_TILE;
-    const int m = min(NBH_DISP_TILE, cnt - base);
-    for (int j = threadIdx.x; j < m; j += 256) {
-        sb[j] = dbin[base + j];
-        for (int q = 0; q < NBH_DISP_Q; ++q) sv[q][j] = dval[(size_t) q * cnt + base + j];
+    for (int j = tid; j < NBH_DISP_TILE; j += 256) {
+        const int i = off + base + j;
+        int bin = -1;
+        if (base + j < cnt && !(ignore && ignore[i])) {
+            const double x = px[i], y = py[i], z = pz[i];
+            double beta;
+            bin = nbh_lambda_beta_bin(h, x, y, z, beta);
+            if (bin >= 0) {
+                const double ux = vx[i], uy = vy[i], uz = vz[i];
+                const double xs = x + h.sun;
+                const double mag = sqrt(xs * xs + y * y + z * z);
+                double mudec, mura;
+                nbh_proper_motion(f, h.sun, x, y, z, ux, uy, uz, mudec, mura);
+                sv[0][j] = beta;
+                sv[1][j] = (xs * ux + y * uy + z * uz) / mag;
+                sv[2][j] = mag;
+                sv[3][j] = mudec;
+                sv[4][j] = mura;
+            }
+        }
+        key[j] = bin >= 0 ? ((unsigned long long) bin << 10) | (unsigned) j : ~0ull;
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nbin; b += 256) {
+    /* bitonic sort of the 1024 keys */
+    for (int k = 2; k <= NBH_DISP_TILE; k <<= 1)
+        for (int d = k >> 1; d > 0; d >>= 1) {
+            for (int t = tid; t < NBH_DISP_TILE / 2; t += 256) {
+                const int i = ((t & ~(d - 1)) << 1) | (t & (d - 1));
+                const unsigned long long a = key[i], b = key[i + d];
+                if ((a > b) == ((i & k) == 0)) {
+                    key[i] = b;
+                    key[i + d] = a;
+                }
+            }
+            __syncthreads();
+        }
+    /* runs of equal bins: four consecutive places a thread */
+    int mine = 0;
+    #pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int p = 4 * tid + u;
+        mine += key[p] != ~0ull && (p == 0 || (key[p - 1] >> 10) != (key[p] >> 10));
+    }
+    int incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o, 64);
+        if ((tid & 63) >= o) incl += y;
+    }
+    if ((tid & 63) == 63) wsum[tid >> 6] = incl;
+    __syncthreads();
+    int at = incl - mine, total = 0;
+    for (int w = 0; w < 4; ++w) {
+        if (w < (tid >> 6)) at += wsum[w];
+        total += wsum[w];
+    }
+    int* start = T.start + (size_t) blockIdx.x * (NBH_DISP_TILE + 1);
+    int* bins = T.bin + (size_t) blockIdx.x * NBH_DISP_TILE;
+    #pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int p = 4 * tid + u;
+        const bool in = key[p] != ~0ull;
+        if (in && (p == 0 || (key[p - 1] >> 10) != (key[p] >> 10))) {
+            start[at] = p;
+            bins[at] = (int) (key[p] >> 10);
+            ++at;
+        }
+        /* the end of the last run: the first place past the binned bodies */
+        if (!in && (p == 0 || key[p - 1] != ~0ull)) start[total] = p;
+        if (in && p == NBH_DISP_TILE - 1) start[total] = NBH_DISP_TILE;
+    }
+    if (tid == 0) T.nrun[blockIdx.x] = total;
+    double* val = T.val + (size_t) blockIdx.x * NBH_DISP_Q * NBH_DISP_TILE;
+    for (int p = tid; p < NBH_DISP_TILE; p += 256) {
+        if (key[p] == ~0ull) continue;
+        const int j = (int) (key[p] & (NBH_DISP_TILE - 1));
+        for (int q = 0; q < NBH_DISP_Q; ++q) val[q * NBH_DISP_TILE + p] = sv[q][j];
+    }
+}
+
+/* One round's sums of a tile.  part is cleared before the first round: a
+ * tile writes only the bins it holds, the same ones every round. */
+__global__ __launch_bounds__(256) void k_disp_part(int nbin, int initial, DispRound r,
+                                                   DispTile T, const double* __restrict__ state,
+                                                   double* __restrict__ part)
+{
+    __shared__ double sv[NBH_DISP_Q][NBH_DISP_TILE];
+    const int nrun = T.nrun[blockIdx.x];
+    if (nrun == 0) return;
+    const int* start = T.start + (size_t) blockIdx.x * (NBH_DISP_TILE + 1);
+    const int* bins = T.bin + (size_t) blockIdx.x * NBH_DISP_TILE;
+    const double* val = T.val + (size_t) blockIdx.x * NBH_DISP_Q * NBH_DISP_TILE;
+    const int m = start[nrun];
+    #pragma unroll
+    for (int q = 0; q < NBH_DISP_Q; ++q)
+        for (int j = threadIdx.x; j < m; j += 256) sv[q][j] = val[q * NBH_DISP_TILE + j];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < NBH_DISP_Q * nrun; idx += 256) {
+        const int q = idx / nrun, run = idx - q * nrun;
+        const int a = start[run], e = start[run + 1], b = bins[run];
         const double* st = state + (size_t) b * NBH_DISP_S;
         /* previous round: mean = sum / (count - removed), sigma = dispersion */
-        double ave[NBH_DISP_Q], cut[NBH_DISP_Q];
-        for (int q = 0; q < NBH_DISP_Q; ++q) {
-            ave[q] = initial ? 0.0 : st[6 * q] / (st[NBH_DISP_RAW] - st[6 * q + 2]);
-            cut[q] = initial ? 0.0 : r.sigma[q] * st[6 * q + 3];
-        }
-        double acc[NBH_DISP_W];
-        for (int w = 0; w < NBH_DISP_W; ++w) acc[w] = 0.0;
-        for (int j = 0; j < m; ++j) {
-            if (sb[j] != b) continue;
-            acc[NBH_DISP_W - 1] += 1.0;
-            for (int q = 0; q < NBH_DISP_Q; ++q) {
-                const double v = sv[q][j];
-                if (initial || fabs(ave[q] - v) < cut[q]) {
-                    acc[3 * q] += v;
-                    acc[3 * q + 1] += v * v;
-                } else {
-                    acc[3 * q + 2] += 1.0;
-                }
+        const double ave = initial ? 0.0 : st[6 * q] / (st[NBH_DISP_RAW] - st[6 * q + 2]);
+        const double cut = initial ? 0.0 : r.sigma[q] * st[6 * q + 3];
+        double sum = 0.0, sq = 0.0, removed = 0.0;
+        #pragma unroll 4
+        for (int j = a; j < e; ++j) {
+            const double v = sv[q][j];
+            if (initial || fabs(ave - v) < cut) {
+                sum += v;
+                sq += v * v;
+            } else {
+                removed += 1.0;
             }
         }
         double* o = part + ((size_t) blockIdx.x * nbin + b) * NBH_DISP_W;
-        for (int w = 0; w < NBH_DISP_W; ++w) o[w] = acc[w];
+        o[3 * q] = sum;
+        o[3 * q + 1] = sq;
+        o[3 * q + 2] = removed;
+        if (q == 0) o[NBH_DISP_W - 1] = (double) (e - a);
     }
 }
 
@@ -263,30 +346,58 @@ __device__ __forceinline__ void nbh_calc_disp(double sum, double sq, double remo
     }
 }
 
-__global__ __launch_bounds__(256) void k_disp_finish(int nbin, int nblk, int initial, DispRound r,
-                                                     const double* __restrict__ part,
-                                                     double* __restrict__ state)
+/* One wave per bin: NBH_DISP_CHUNK tiles' sums are staged in LDS (the next
+ * chunk's loads in flight meanwhile), and a lane per sum adds them in tile
+ * order. */
+#define NBH_DISP_CHUNK 32
+__global__ __launch_bounds__(64) void k_disp_finish(int nbin, int nblk, int initial, DispRound r,
+                                                    const double* __restrict__ part,
+                                                    double* __restrict__ state)
 {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= nbin) return;
-    double t[NBH_DISP_W];
-    for (int w = 0; w < NBH_DISP_W; ++w) t[w] = 0.0;
-    for (int k = 0; k < nblk; ++k) {
-        const double* o = part + ((size_t) k * nbin + b) * NBH_DISP_W;
-        for (int w = 0; w < NBH_DISP_W; ++w) t[w] += o[w];
+    constexpr int L = NBH_DISP_CHUNK * NBH_DISP_W / 64;      /* loads per lane and chunk */
+    __shared__ double buf[NBH_DISP_CHUNK * NBH_DISP_W];
+    __shared__ double t[NBH_DISP_W];
+    const int b = blockIdx.x;
+    const int lane = threadIdx.x;
+    double next[L];
+    auto fetch = [&](int k0) {
+        #pragma unroll
+        for (int u = 0; u < L; ++u) {
+            const int e = u * 64 + lane;
+            const int k = k0 + e / NBH_DISP_W;
+            next[u] = k < nblk ? part[((size_t) k * nbin + b) * NBH_DISP_W + e % NBH_DISP_W] : 0.0;
+        }
+    };
+    fetch(0);
+    double acc = 0.0;
+    for (int k0 = 0; k0 < nblk; k0 += NBH_DISP_CHUNK) {
+        #pragma unroll
+        for (int u = 0; u < L; ++u) buf[u * 64 + lane] = next[u];
+        __syncthreads();
+        if (k0 + NBH_DISP_CHUNK < nblk) fetch(k0 + NBH_DISP_CHUNK);
+        if (lane < NBH_DISP_W) {
+            const int c = min(NBH_DISP_CHUNK, nblk - k0);
+            #pragma unroll 8
+            for (int k = 0; k < c; ++k) acc += buf[k * NBH_DISP_W + lane];
+        }
+        __syncthreads();
     }
+    if (lane < NBH_DISP_W) t[lane] = acc;
+    __syncthreads();
+    if (lane >= NBH_DISP_Q) return;
+    const int q = lane;
     double* st = state + (size_t) b * NBH_DISP_S;
-    st[NBH_DISP_RAW] = t[NBH_DISP_W - 1];
-    for (int q = 0; q < NBH_DISP_Q; ++q) {
-        double* sq = st + 6 * q;
-        /* every bin starts at dispersion 0 (nbody_histogram.c:846-854) */
-        if (initial) sq[3] = sq[4] = 0.0;
-        sq[0] = t[3 * q];
-        sq[1] = t[3 * q + 1];
-        sq[2] = t[3 * q + 2];
-        nbh_calc_disp(sq[0], sq[1], sq[2], st[NBH_DISP_RAW], initial, r.correct[q], sq[3],
-                      sq[4]);
-    }
+    if (q == 0) st[NBH_DISP_RAW] = t[NBH_DISP_W - 1];
+    double* sq = st + 6 * q;
+    /* every bin starts at dispersion 0 (nbody_histogram.c:846-854) */
+    double var = initial ? 0.0 : sq[3], err = initial ? 0.0 : sq[4];
+    nbh_calc_disp(t[3 * q], t[3 * q + 1], t[3 * q + 2], t[NBH_DISP_W - 1], initial, r.correct[q],
+                  var, err);
+    sq[0] = t[3 * q];
+    sq[1] = t[3 * q + 1];
+    sq[2] = t[3 * q + 2];
+    sq[3] = var;
+    sq[4] = err;
 }
 
 /* Histograms 1-7 from the final state: dispersions of beta and v_los, and
@@ -323,10 +434,41 @@ __global__ __launch_bounds__(256) void k_disp_out(int nbin, const double* __rest
 static inline int nbh_blocks(int n, int per) { return n > 0 ? (n + per - 1) / per : 1; }
 
 static HistParams nbh_hist_params(const nbhip_histogram_params* hp);
+__global__ void k_fill_u32(unsigned* __restrict__ p, size_t n, unsigned v);
 
-void nbh_dispersion(nbhip_state* st, int off, int cnt, const nbhip_histogram_params* hp,
-                    const nbhip_disp_params* dp, int* dbin, double* dval, double* part,
-                    double* state, double* out)
+/* Sections of the dispersions' scratch, each 256-byte aligned: the tiles'
+ * values, runs and run counts, the per-tile partial sums, the per-bin state
+ * and the output rows. */
+struct DispScratch {
+    size_t val, start, bin, nrun, part, state, out, total;
+};
+static DispScratch nbh_disp_layout(size_t nblk, size_t nbin)
+{
+    DispScratch d;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) & ~(size_t) 255;
+        return o;
+    };
+    d.val = take(nblk * NBH_DISP_Q * NBH_DISP_TILE * sizeof(double));
+    d.start = take(nblk * (NBH_DISP_TILE + 1) * sizeof(int));
+    d.bin = take(nblk * NBH_DISP_TILE * sizeof(int));
+    d.nrun = take(nblk * sizeof(int));
+    d.part = take(nblk * nbin * NBH_DISP_W * sizeof(double));
+    d.state = take(nbin * NBH_DISP_S * sizeof(double));
+    d.out = take(14 * nbin * sizeof(double));
+    d.total = at;
+    return d;
+}
+
+size_t nbh_disp_bytes(int cnt, size_t nbin)
+{
+    return nbh_disp_layout(((size_t) cnt + NBH_DISP_TILE - 1) / NBH_DISP_TILE, nbin).total;
+}
+
+const double* nbh_dispersion(nbhip_state* st, int off, int cnt, const nbhip_histogram_params* hp,
+                             const nbhip_disp_params* dp, char* scratch_bytes)
 {
     const HistParams h = nbh_hist_params(hp);
     const int nbin = hp->lambda_bins * hp->beta_bins;
@@ -349,19 +491,31 @@ void nbh_dispersion(nbhip_state* st, int off, int cnt, const nbhip_histogram_par
     f.rot[1][0] = sa * cd * cl + ca * sl; f.rot[1][1] = -sa * cd * sl + ca * cl; f.rot[1][2] = sa * sd;
     f.rot[2][0] = -sd * cl; f.rot[2][1] = sd * sl; f.rot[2][2] = cd;
     for (int k = 0; k < 3; ++k) f.sun_vel[k] = dp->sun_vel[k];
+    const DispScratch d = nbh_disp_layout((size_t) nblk, (size_t) nbin);
+    char* base = scratch_bytes;
+    const DispTile T = { reinterpret_cast<double*>(base + d.val),
+                         reinterpret_cast<int*>(base + d.start),
+                         reinterpret_cast<int*>(base + d.bin),
+                         reinterpret_cast<int*>(base + d.nrun) };
+    double* part = reinterpret_cast<double*>(base + d.part);
+    double* state = reinterpret_cast<double*>(base + d.state);
+    double* out = reinterpret_cast<double*>(base + d.out);
     hipStream_t s = st->stream;
-    hipLaunchKernelGGL(k_disp_values, dim3(nbh_blocks(cnt, 256)), dim3(256), 0, s, off, cnt,
-                       st->px, st->py, st->pz, st->vx, st->vy, st->vz, st->ignore, h, f, dbin,
-                       dval);
+    hipLaunchKernelGGL(k_disp_values, dim3(nblk), dim3(256), 0, s, off, cnt, st->px, st->py,
+                       st->pz, st->vx, st->vy, st->vz, st->ignore, h, f, T);
+    const size_t words = (size_t) nblk * nbin * NBH_DISP_W * 2;
+    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned) std::min<size_t>((words + 255) / 256, 4096)),
+                       dim3(256), 0, s, reinterpret_cast<unsigned*>(part), words, 0u);
     for (int round = 0; round <= dp->iter_max; ++round) {
         const int initial = round == 0;
-        hipLaunchKernelGGL(k_disp_part, dim3(nblk), dim3(256), 0, s, cnt, nbin, initial, r,
-                           dbin, dval, state, part);
-        hipLaunchKernelGGL(k_disp_finish, dim3(nbh_blocks(nbin, 256)), dim3(256), 0, s, nbin,
-                           nblk, initial, r, part, state);
+        hipLaunchKernelGGL(k_disp_part, dim3(nblk), dim3(256), 0, s, nbin, initial, r, T, state,
+                           part);
+        hipLaunchKernelGGL(k_disp_finish, dim3(nbin), dim3(64), 0, s, nbin, nblk, initial, r,
+                           part, state);
     }
     hipLaunchKernelGGL(k_disp_out, dim3(nbh_blocks(nbin, 256)), dim3(256), 0, s, nbin, state,
                        out);
+    return out;
 }
 
 static HistParams nbh_hist_params(const nbhip_histogram_params* hp)
@@ -387,8 +541,13 @@ void nbh_histogram(nbhip_state* st, const nbhip_histogram_params* hp, unsigned* 
                    unsigned* d_totals)
 {
     const HistParams h = nbh_hist_params(hp);
-    hipLaunchKernelGGL(k_histogram, dim3(nbh_blocks(st->n, 256)), dim3(256), 0, st->stream,
-                       st->n, st->px, st->py, st->pz, st->ignore, st->simid, h, d_counts,
+    /* each workgroup adds its non-empty bins to the same few counters, so one
+     * simulation takes eight bodies a thread once that still fills the chip
+     * (10^6 bodies, 50 bins: 35 -> 19 us); a batch keeps one, so that few
+     * workgroups straddle two simulations */
+    const int per = st->nsim == 1 && st->n >= 256 * 256 * 8 ? 8 : 1;
+    hipLaunchKernelGGL(k_histogram, dim3(nbh_blocks(st->n, 256 * per)), dim3(256), 0, st->stream,
+                       st->n, st->px, st->py, st->pz, st->ignore, st->simid, h, per, d_counts,
                        d_totals);
 }
 

@@ -279,9 +279,9 @@ void nbh_walk_group(nbhip_state* st, const WalkOut& o, double* out_ax, double* o
 /* launcher (histogram.hip) */
 void nbh_histogram(nbhip_state* st, const nbhip_histogram_params* hp, unsigned* d_counts,
                    unsigned* d_totals);
-void nbh_dispersion(nbhip_state* st, int off, int cnt, const nbhip_histogram_params* hp,
-                    const nbhip_disp_params* dp, int* dbin, double* dval, double* part,
-                    double* state, double* out);
+size_t nbh_disp_bytes(int cnt, size_t nbin);
+const double* nbh_dispersion(nbhip_state* st, int off, int cnt, const nbhip_histogram_params* hp,
+                             const nbhip_disp_params* dp, char* scratch_bytes);
 /* scratch of the allocation-free entry point (histogram.hip) */
 unsigned nbh_scratch_init(int device);
 /* launchers (adjoint.hip) */
