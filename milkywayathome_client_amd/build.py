@@ -23,7 +23,7 @@ MODELS_LIB_PATH = os.path.join(PKG_DIR, "libnbmodels.so")
 # other sources is refused, not used).
 STAMP_PATH = os.path.join(PKG_DIR, "libnbhip.srchash")
 
-SOURCES = ["api.hip", "tree.hip", "walk.hip", "walk_group.hip", "adjoint.hip", "histogram.hip",
+SOURCES = ["api.hip", "tree.hip", "walk.hip", "walk_group.hip", "walk_list.hip", "adjoint.hip", "histogram.hip",
            "exact.hip", "run.hip", "checkpoint.hip", "dwarf.hip"]
 
 # -ffp-contract=off: the plain FP64 form keeps the reference's two-rounding

@@ -106,7 +106,8 @@ static void nbh_free_all(nbhip_state* st)
                      st->scal, st->sims, st->ignore, st->hist_buf, st->disp_buf, st->pos4,
                      st->exact_part, st->nodeg, st->nkid, st->kbase, st->best_buf,
                      st->nrank, st->kid, st->blist, st->span, st->span_sorted, st->gcost,
-                     st->gorder, st->bcost, st->gtask, st->nnext, st->bbox };
+                     st->gorder, st->bcost, st->gtask, st->nnext, st->bbox,
+                     st->wlist, st->wlen };
     for (void* p : ptrs)
         if (p) (void) hipFree(p);
     if (st->graph_exec) (void) hipGraphExecDestroy(st->graph_exec);
@@ -225,6 +226,12 @@ static unsigned nbh_create(const nbhip_ctx* ctx, int device, int nsim, const int
         /* the first walk has no costs yet: all zero, so every group in one bucket */
         if (e == hipSuccess) e = hipMemset(st->bcost, 0, (n ? n : 1) * sizeof(unsigned));
         if (e == hipSuccess) e = hipMemset(st->bbox, 0, (n ? n : 1) * sizeof(float));
+    }
+    if (ctx->precision == NBHIP_PRECISION_FP64 && ctx->criterion != NBHIP_EXACT &&
+        st->n <= NBH_LIST_BODIES) {
+        const size_t ng = ((size_t) st->n + 63) / 64 + 1;
+        A(wlist, ng * NBH_LIST_CAP);
+        A(wlen, ng);
     }
     A(nkid, nc); A(kbase, nc); A(nrank, nc); A(kid, nc); A(blist, nc); A(span, nc);
     A(span_sorted, nc);

@@ -359,6 +359,13 @@ __device__ __forceinline__ unsigned long long nbh_lanemask_lt()
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
+/* Set bits of m below this lane. */
+__device__ __forceinline__ unsigned nbh_mbcnt(unsigned long long m)
+{
+    return __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+}
+
 __device__ __forceinline__ double nbh_wave_max(double v)
 {
     for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));

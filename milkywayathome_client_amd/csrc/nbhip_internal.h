@@ -149,6 +149,14 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
     return at + 16;
 }
 
+/* Interaction lists of the FP64 list walk: entries per 64-body group (LDS of
+ * the list's build: 8 bytes an entry). */
+#define NBH_LIST_CAP 8192
+/* states of at most this many bodies walk lists (walk_list.hip has both
+ * sides' times), and of at most this many with sixteen entries a batch */
+#define NBH_LIST_BODIES (1 << 17)
+#define NBH_LIST_WIDE 8192
+
 #define NBH_SORT_TILE 2048   /* keys per radix-sort block: 256 threads x 8 */
 #define NBH_SCAN_TILE 4096   /* items per scan block: 1024 threads x 4 */
 
@@ -221,6 +229,8 @@ struct nbhip_state {
     int *kid;                     /* child lists: kid[kbase[p] .. + nkid[p]) */
     int *blist;                   /* summaries: inside cells of each body block, by level */
     int *span, *span_sorted;      /* summaries: cells spanning body blocks / super-blocks */
+    int *wlist, *wlen;            /* FP64 list walk: each 64-body group's nodes in pre-order
+                                     (NBH_LIST_CAP slots) and their count, -1: streaming walk */
     double *exact_part;           /* Exact criterion: per-segment partial sums */
     int exact_seg;                /* Exact criterion: most segments of any simulation */
 
@@ -271,6 +281,8 @@ void nbh_masses_changed(nbhip_state* st);
 /* launchers (walk.hip) */
 void nbh_walk(nbhip_state* st, int kick, int count, double* out_ax, double* out_ay,
               double* out_az, int self_only, const WalkTune* tune);
+void nbh_walk_list(nbhip_state* st, const struct WalkOut& o, double* out_ax, double* out_ay,
+                   double* out_az);
 void nbh_direct(nbhip_state* st, int nsample, const int* d_idx, double* d_acc);
 /* launcher (walk_group.hip) */
 struct WalkOut;

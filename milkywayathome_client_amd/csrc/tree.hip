@@ -1063,6 +1063,7 @@ __global__ __launch_bounds__(256) void k_emit_leaves(int n, const int* __restric
                                                      int* __restrict__ nsim,
                                                      SimTab* __restrict__ sims,
                                                      NodeF* __restrict__ nodef,
+                                                     double* __restrict__ nquad,
                                                      unsigned* __restrict__ nkid,
                                                      int* __restrict__ nrank,
                                                      int* __restrict__ nnext,
@@ -1113,6 +1114,10 @@ __global__ __launch_bounds__(256) void k_emit_leaves(int n, const int* __restric
     nlevel[pre] = -1;
     nparent[pre] = parent;
     nsim[pre] = sim;
+    if (nquad) {                       /* the list walk reads a body's like a cell's */
+        double2* q = reinterpret_cast<double2*>(nquad + 6 * (size_t) pre);
+        q[0] = q[1] = q[2] = make_double2(0.0, 0.0);
+    }
     if (nodef) {
         NodeF f;
         f.x = p.x;
@@ -1949,8 +1954,8 @@ void nbh_build(nbhip_state* st, int graph_safe)
                        st->sims, st->nkid, st->nrank, st->nnext, st->scal);
     hipLaunchKernelGGL(k_emit_leaves, dim3(g256), dim3(256), 0, s, n, st->dadj, st->su, st->cincl,
                        st->spos, st->simid_s, st->node, st->nmid, st->nlevel, st->nparent,
-                       st->nsim_node, st->sims, st->nodef, st->nkid, st->nrank, st->nnext,
-                       st->scal);
+                       st->nsim_node, st->sims, st->nodef, st->wlist ? st->nquad : nullptr,
+                       st->nkid, st->nrank, st->nnext, st->scal);
     /* each cell's child block (kbase) and child list (kid) */
     const int nt = nbh_blocks(st->node_cap, NBH_SCAN_TILE);
     hipLaunchKernelGGL(k_nscan_tiles, dim3(nt), dim3(1024), 0, s, st->nkid, st->kbase,

@@ -82,12 +82,6 @@ __device__ __forceinline__ int nbh_wave_min_u(int v)
     return __builtin_amdgcn_readfirstlane(nbh_wave_min_i(v));
 }
 
-__device__ __forceinline__ unsigned nbh_mbcnt(unsigned long long m)
-{
-    return __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-}
-
 /* Cuts of one wave: bit i set = a sub-group ends at lane i.  `lvl` is the
  * level of the common prefix of this lane's body and the next lane's (-1
  * where the next lane is in another simulation, massless, invalid or past

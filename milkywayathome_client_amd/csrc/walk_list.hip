@@ -1,0 +1,583 @@
+/*
+ * FP64 walk from interaction lists (plain form, precision NBHIP_PRECISION_FP64)
+ * on gfx950, for states too small to fill the chip with one lane per body.
+ *
+ * The streaming walk (walk.hip) is a serial chain per wavefront of 64 bodies:
+ * a scalar load, the test, the wave's vote, the branch, and an interaction
+ * whose square root and quotients depend on each other, some 1200 cycles a
+ * node step and 2000-3500 steps.  20 000 bodies are 313 such wavefronts on
+ * 1024 SIMDs: 1.5 ms, of which the arithmetic fills a tenth.  Here the chain
+ * is cut in two:
+ *
+ *  1. k_list_build, a workgroup per 64 consecutive sorted bodies, finds every
+ *     node that any of them can meet, breadth first (all nodes of a level at
+ *     once): a node is decided by the bodies' bounding box where its nearest
+ *     point already passes the test (every body accepts) or its farthest point
+ *     fails it (every body opens), and by the 64 tests themselves otherwise.
+ *     Nodes that some body accepts are the list; it is put into pre-order
+ *     (subtree sizes up the levels, places down them).
+ *  2. k_walk_list, a wavefront per 8 (or 4) bodies, goes through the list in
+ *     order: 64 entries at a time are tested against its own bodies, those
+ *     that none of them accepts or that lie inside one accepted by all are
+ *     dropped, and the others are taken 8 (16) at a time: lane (b, s) tests
+ *     and evaluates entry s for body b.
+ *
+ * The reference's walk (nbGravity, nbody/src/nbody_grav.c:42-124) is kept to
+ * the bit: the box only replaces decisions that are the same for every body
+ * (rounding is monotone, so a box's nearest and farthest point bound the
+ * computed squared distances of the bodies in it), a body's own test decides
+ * the rest, a body skips what lies inside a node it has accepted (its place
+ * in the walk, lp, as in the streaming walk), and its terms are added in
+ * pre-order: the lanes leave their nine terms in LDS and one lane per (body,
+ * component) adds them entry by entry, the reference's three additions each;
+ * a lane that does not interact leaves zeros, which change no bit of the sum.
+ *
+ * A group whose nodes do not fit the list (NBH_LIST_CAP) is left to the
+ * streaming walk, which runs after this one over such groups only.
+ *
+ * Measured (lists + walk against the streaming walk, BH86 theta = 0.5 with
+ * quadrupoles): 1000 bodies 120 : 386 us, 4000 202 : 890, 20 000 413 : 1520,
+ * 50 000 1024 : 1795, 100 000 1970 : 2445, 200 000 4200 : 3460 -- so up to
+ * NBH_LIST_BODIES (131 072).  At 20 000 bodies the walk is 335 us (its
+ * vector instructions alone 170) and the lists 79.  Beyond, each SIMD has
+ * enough streaming waves to hide their chain, and the lists' LDS traffic
+ * (17 LDS instructions per batch) no longer pays.
+ */
+#include "nbhip_walk.h"
+
+#include <type_traits>
+
+#define NBH_LIST_KEEP (1u << 31)      /* build entry: goes into the list */
+#define NBH_LIST_OPEN (1u << 30)      /* its children are entries too */
+#define NBH_LIST_Q ((1u << 27) - 1u)  /* pre-order index; bits 27..29: children - 1 */
+
+/* Squared distances from a node to the nearest and the farthest point of a
+ * box, in the walk's operation order. */
+struct ListBox {
+    double lox, loy, loz, hix, hiy, hiz;
+    __device__ __forceinline__ void dist(double x, double y, double z, double& near2,
+                                         double& far2) const
+    {
+        const double ax = lox - x, bx = x - hix, ay = loy - y, by = y - hiy, az = loz - z,
+                     bz = z - hiz;
+        const double nx = fmax(fmax(ax, bx), 0.0), ny = fmax(fmax(ay, by), 0.0),
+                     nz = fmax(fmax(az, bz), 0.0);
+        const double fx = fmax(fabs(ax), fabs(bx)), fy = fmax(fabs(ay), fabs(by)),
+                     fz = fmax(fabs(az), fabs(bz));
+        near2 = nz * nz + (ny * ny + nx * nx);
+        far2 = fz * fz + (fy * fy + fx * fx);
+    }
+};
+
+__device__ __forceinline__ double nbh_wmin(double v)
+{
+    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
+    return v;
+}
+
+/* The box of the wave's valid bodies. */
+__device__ __forceinline__ ListBox nbh_list_box(bool valid, const double4& p)
+{
+    ListBox b;
+    b.lox = nbh_wmin(valid ? p.x : INFINITY);
+    b.loy = nbh_wmin(valid ? p.y : INFINITY);
+    b.loz = nbh_wmin(valid ? p.z : INFINITY);
+    b.hix = nbh_wave_max(valid ? p.x : -INFINITY);
+    b.hiy = nbh_wave_max(valid ? p.y : -INFINITY);
+    b.hiz = nbh_wave_max(valid ? p.z : -INFINITY);
+    return b;
+}
+
+/* Interaction list of each 64-body group: list[g * NBH_LIST_CAP ..), length
+ * llen[g], -1 where it does not fit.  All waves hold the group's bodies
+ * (lane = body) for the box and share the nodes of a level. */
+#define NBH_LB 512                    /* threads of k_list_build */
+__global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__ node,
+                                                    const double4* __restrict__ spos,
+                                                    const int* __restrict__ simid_s,
+                                                    const SimTab* __restrict__ sims,
+                                                    const unsigned* __restrict__ nkid,
+                                                    const unsigned* __restrict__ kbase,
+                                                    const int* __restrict__ kid,
+                                                    int* __restrict__ list,
+                                                    int* __restrict__ llen,
+                                                    const DevScalars* __restrict__ scal, int n,
+                                                    int multi)
+{
+    __shared__ unsigned s_q[NBH_LIST_CAP];            /* entry: flags and pre-order index */
+    __shared__ unsigned short s_c[NBH_LIST_CAP];      /* first child's entry */
+    __shared__ unsigned short s_n[NBH_LIST_CAP];      /* list entries in the subtree, then place */
+    __shared__ int s_lev[65];                         /* first entry of each level */
+    __shared__ double4 s_body[64];
+    __shared__ int s_cnt, s_over, s_mix;
+    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int g = blockIdx.x;
+    const int s = g * 64 + lane;
+    const bool valid = s < n;
+    const double4 p = valid ? spos[s] : make_double4(0.0, 0.0, 0.0, 0.0);
+    const ListBox box = nbh_list_box(valid, p);
+    const int sim = valid ? simid_s[s] : -1;
+    if (tid < 64) s_body[tid] = p;
+    if (tid == 0) {
+        s_cnt = 0;
+        s_over = 0;
+    }
+    __syncthreads();
+    /* the roots of the group's simulations, in pre-order */
+    if (!multi) {
+        if (tid == 0 && sims[0].root >= 0) {
+            s_q[0] = (unsigned) sims[0].root;
+            s_cnt = 1;
+        }
+    } else if (tid < 64) {
+        const int root = valid ? sims[sim].root : -1;
+        bool first = root >= 0;
+        for (int k = 1; k < 64; ++k) {
+            const int o = __shfl(root, lane >= k ? lane - k : 0, 64);
+            if (lane >= k && o == root) first = false;
+        }
+        const unsigned long long fm = __builtin_amdgcn_ballot_w64(first);
+        int at = 0;
+        for (unsigned long long r = fm; r; r &= r - 1)
+            at += __builtin_amdgcn_readlane(root, __builtin_ctzll(r)) < root;
+        if (first) s_q[at] = (unsigned) root;
+        if (lane == 0) s_cnt = __popcll(fm);
+    }
+    __syncthreads();
+    int lo = 0, hi = s_cnt, depth = 0;
+    const int nroot = hi;
+    const int nb = min(64, n - g * 64);
+    /* entry i decided: kept or not, and its children's entries (all eight
+     * loads of the child list in flight at once) */
+    auto decide = [&](int i, unsigned q, bool open, bool keep, unsigned mask, unsigned kb) {
+        unsigned e = q | (keep ? NBH_LIST_KEEP : 0u);
+        if (open) {
+            const int nk = __popc(mask);
+            const int at = atomicAdd(&s_cnt, nk);
+            if (at + nk > NBH_LIST_CAP || nk < 1 || nk > 8) {
+                s_over = 1;
+            } else {
+                e |= NBH_LIST_OPEN | (unsigned) (nk - 1) << 27;
+                s_c[i] = (unsigned short) at;
+                int ch[8];
+                #pragma unroll
+                for (int j = 0; j < 8; ++j) ch[j] = kid[kb + min(j, nk - 1)];
+                #pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (j < nk) s_q[at + j] = (unsigned) ch[j];
+            }
+        }
+        s_q[i] = e;
+    };
+    while (lo < hi && depth < 64) {
+        if (tid == 0) {
+            s_lev[depth] = lo;
+            s_mix = 0;
+        }
+        __syncthreads();
+        /* what the group's box decides for every body; the rest to the work
+         * list (s_n is free until the subtrees are counted) */
+        for (int i = lo + tid; i < hi; i += NBH_LB) {
+            const unsigned q = s_q[i];
+            const NodeW w = node[q];
+            const unsigned mask = nkid[q], kb = kbase[q];
+            double near2, far2;
+            box.dist(w.x, w.y, w.z, near2, far2);
+            const bool cell = w.body < 0;
+            if (!cell || near2 >= w.rcrit2) decide(i, q, false, true, mask, kb);
+            else if (far2 < w.rcrit2) decide(i, q, true, false, mask, kb);
+            else s_n[atomicAdd(&s_mix, 1)] = (unsigned short) i;
+        }
+        __syncthreads();
+        /* the bodies' own tests, four lanes a node */
+        const int nmix = s_mix;
+        for (int t = tid; t < 4 * nmix; t += NBH_LB) {
+            const int i = s_n[t >> 2];
+            const unsigned q = s_q[i];
+            const NodeW w = node[q];
+            const unsigned mask = nkid[q], kb = kbase[q];
+            int seen = 0;                             /* 1: a body accepts, 2: a body opens */
+            #pragma unroll 4
+            for (int k = t & 3; k < nb; k += 4) {
+                const double4 c = s_body[k];
+                const double dx = w.x - c.x, dy = w.y - c.y, dz = w.z - c.z;
+                seen |= dz * dz + (dy * dy + dx * dx) >= w.rcrit2 ? 1 : 2;
+            }
+            seen |= __builtin_amdgcn_mov_dpp(seen, 0xB1, 0xF, 0xF, true);
+            seen |= __builtin_amdgcn_mov_dpp(seen, 0x4E, 0xF, 0xF, true);
+            if ((t & 3) == 0) decide(i, q, (seen & 2) != 0, (seen & 1) != 0, mask, kb);
+        }
+        __syncthreads();
+        if (s_over) {
+            if (tid == 0) llen[g] = -1;
+            return;
+        }
+        lo = hi;
+        hi = s_cnt;
+        ++depth;
+        __syncthreads();
+    }
+    if (lo < hi) {                    /* deeper than 63 levels: not a tree of ours */
+        if (tid == 0) llen[g] = -1;
+        return;
+    }
+    if (tid == 0) s_lev[depth] = hi;
+    __syncthreads();
+    /* list entries of each subtree, deepest level first */
+    for (int l = depth - 1; l >= 0; --l) {
+        for (int i = s_lev[l] + tid; i < s_lev[l + 1]; i += NBH_LB) {
+            const unsigned e = s_q[i];
+            int c = (e & NBH_LIST_KEEP) ? 1 : 0;
+            if (e & NBH_LIST_OPEN) {
+                const int a = s_c[i], nk = (int) ((e >> 27) & 7u) + 1;
+                for (int j = 0; j < nk; ++j) c += s_n[a + j];
+            }
+            s_n[i] = (unsigned short) c;
+        }
+        __syncthreads();
+    }
+    /* places, from the roots down; a kept entry writes itself */
+    int* out = list + (size_t) g * NBH_LIST_CAP;
+    if (tid == 0) {
+        int at = 0;
+        for (int r = 0; r < nroot; ++r) {
+            const int c = s_n[r];
+            s_n[r] = (unsigned short) at;
+            at += c;
+        }
+        llen[g] = at;
+    }
+    __syncthreads();
+    for (int l = 0; l < depth; ++l) {
+        for (int i = s_lev[l] + tid; i < s_lev[l + 1]; i += NBH_LB) {
+            const unsigned e = s_q[i];
+            int at = s_n[i];
+            if (e & NBH_LIST_KEEP) out[at++] = (int) (e & NBH_LIST_Q);
+            if (e & NBH_LIST_OPEN) {
+                const int a = s_c[i], nk = (int) ((e >> 27) & 7u) + 1;
+                for (int j = 0; j < nk; ++j) {
+                    const int c = s_n[a + j];
+                    s_n[a + j] = (unsigned short) at;
+                    at += c;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+/* Maximum over the S = 4, 8 or 16 consecutive lanes of a body. */
+template <int S>
+__device__ __forceinline__ int nbh_slots_max(int v)
+{
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true));              /* xor 1 */
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true));              /* xor 2 */
+    if (S >= 8) v = max(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true)); /* half row mirrored */
+    if (S >= 16) v = max(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true)); /* row mirrored */
+    return v;
+}
+
+/* v of one lane, uniform. */
+__device__ __forceinline__ double nbh_lane_d(double v, int lane)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int) (unsigned) (b & 0xffffffffll), lane);
+    const int hi = __builtin_amdgcn_readlane((int) (b >> 32), lane);
+    return __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
+}
+
+#define NBH_LIST_RING 128
+
+/* A batch lane's node: record and quadrupole as loaded; cont has bit S - d
+ * set where the entry d places back contains this one. */
+struct ListRec {
+    unsigned q, cont;
+    double2 xy, zm, rl, q0, q1, q2;
+};
+
+/* Maximum over this lane and the lanes below it. */
+__device__ __forceinline__ int nbh_scan_max(int v)
+{
+    /* row_shr 1, 2, 4, 8, then each row's last lane to the rows above
+     * (lanes without a source read 0: the values are indices >= 0) */
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false)); /* row_bcast 15 */
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false)); /* row_bcast 31 */
+    return v;
+}
+
+/* The terms in LDS: [component][term][lane], a write being one run of 64
+ * doubles; the second half of the lanes two doubles on and rows of 76, which
+ * keeps the adders' 16-byte reads (a body's slots, three components) on
+ * different banks. */
+#define NBH_TERM_ROW 76
+__device__ __forceinline__ int nbh_term_at(int c, int t, int T, int lane)
+{
+    return (c * T + t) * NBH_TERM_ROW + lane + (lane >= 32 ? 2 : 0);
+}
+
+/* lane = b * S + s: body b of the wave's B = 64 / S, slot s of the batch. */
+#define NBH_LW 2                      /* wavefronts per workgroup of k_walk_list */
+template <int S, bool QUAD>
+__global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restrict__ node,
+                                                   const double* __restrict__ nquad,
+                                                   const double4* __restrict__ spos,
+                                                   const unsigned* __restrict__ perm,
+                                                   const int* __restrict__ simid_s,
+                                                   SimTab* __restrict__ sims,
+                                                   const int* __restrict__ list,
+                                                   const int* __restrict__ llen,
+                                                   double* __restrict__ oax,
+                                                   double* __restrict__ oay,
+                                                   double* __restrict__ oaz,
+                                                   double* __restrict__ vx,
+                                                   double* __restrict__ vy,
+                                                   double* __restrict__ vz,
+                                                   DevScalars* __restrict__ scal, WalkOut o)
+{
+    constexpr int B = 64 / S;
+    constexpr int T = QUAD ? 3 : 1;                   /* additions per component and entry */
+    __shared__ int2 s_ring[NBH_LW][NBH_LIST_RING];         /* pre-order index, containing entries */
+    __shared__ int s_next[NBH_LW][NBH_LIST_RING];
+    __shared__ __align__(16) double s_term[NBH_LW][3 * T * NBH_TERM_ROW];
+    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    const int w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int b = lane / S, slot = lane % S;
+    const int first = (blockIdx.x * NBH_LW + w) * B;       /* the wave's first body */
+    if (first >= o.n) return;
+    const int g = first >> 6;
+    const int len = llen[g];
+    if (len < 0) return;                              /* the streaming walk's */
+    const int* lst = list + (size_t) g * NBH_LIST_CAP;
+    int2* ring = s_ring[w];
+    int* rnext = s_next[w];
+    double* term = s_term[w];
+    const int body = first + b;
+    const bool valid = body < o.n;
+    const double4 p = valid ? spos[body] : make_double4(0.0, 0.0, 0.0, 0.0);
+    /* the wave's bodies, uniform, for the filter (past the end: the first) */
+    double bx[B], by[B], bz[B];
+    {
+        const double4 f = spos[first];
+        const double vx_ = valid ? p.x : f.x, vy_ = valid ? p.y : f.y, vz_ = valid ? p.z : f.z;
+        #pragma unroll
+        for (int k = 0; k < B; ++k) {
+            bx[k] = nbh_lane_d(vx_, k * S);
+            by[k] = nbh_lane_d(vy_, k * S);
+            bz[k] = nbh_lane_d(vz_, k * S);
+        }
+    }
+    const int sim = valid ? simid_s[body] : simid_s[first];
+    const SimTab& st = sims[sim];
+    const double eps2 = st.eps2;
+    int lp = valid && st.root >= 0 ? st.root : INT_MAX;
+    const int end = o.multi ? st.end : INT_MAX;
+    const int self = valid && body < scal->nmassive ? body : -2;
+    const bool eps2_pos = o.all_eps2_pos;
+    const bool plain = __builtin_amdgcn_ballot_w64(!nbh_plain_range(st)) == 0ull;
+    bool met = false;
+    double acc = 0.0;                                 /* of body lane % B, component lane / B */
+    rnext[lane] = 0;
+    rnext[lane + 64] = 0;
+    ring[lane] = ring[lane + 64] = make_int2(0, 0);
+
+    /* entries head .. head + S - 1 of the ring */
+    auto fetch = [&](int head, int cnt) {
+        ListRec r;
+        const int2 e = ring[(head + slot) & (NBH_LIST_RING - 1)];
+        r.q = slot < cnt ? (unsigned) e.x : 0u;
+        r.cont = (unsigned) e.y;
+        /* 32-bit offsets: a state with lists has under 2^21 nodes */
+        const unsigned off = r.q * 48u;
+        const double2* rec =
+            reinterpret_cast<const double2*>(reinterpret_cast<const char*>(node) + off);
+        r.xy = rec[0];
+        r.zm = rec[1];
+        r.rl = rec[2];
+        if (QUAD) {
+            const double2* qr =
+                reinterpret_cast<const double2*>(reinterpret_cast<const char*>(nquad) + off);
+            r.q0 = qr[0];
+            r.q1 = qr[1];
+            r.q2 = qr[2];
+        }
+        return r;
+    };
+    /* one batch, `cnt` of its entries live */
+    auto batch = [&](const ListRec& r, int cnt) {
+        const bool live = slot < cnt;
+        const unsigned q = r.q;
+        const double2 xy = r.xy, zm = r.zm, rl = r.rl;
+        const long long link = __double_as_longlong(rl.y);
+        const int next = (int) (unsigned) (link & 0xffffffffll);
+        const int nbody = (int) (link >> 32);
+        const double dx = xy.x - p.x, dy = xy.y - p.y, dz = zm.x - p.z;
+        const double drSq = dz * dz + (dy * dy + dx * dx);
+        /* a node passes by itself; it is met unless it lies inside one that
+         * was accepted: before this batch (lp) or in it (cont) */
+        const bool pass = live & (drSq >= rl.x);      /* a body's rcrit2 is 0 */
+        const unsigned long long pm = __builtin_amdgcn_ballot_w64(pass);
+        const unsigned mine = (unsigned) (pm >> (b * S)) << (S - slot);
+        const bool met_here = pass & ((int) q >= lp) & ((int) q < end) & ((mine & r.cont) == 0u);
+        lp = max(lp, nbh_slots_max<S>(pass ? next : 0));
+        met |= met_here & (nbody == self);
+        const bool use = met_here & (eps2_pos | (nbody != self));
+        /* unused lanes: mass 0 and no quadrupole, at a harmless distance */
+        const double r2 = use ? drSq + eps2 : 1.0;
+        const double m = use ? zm.y : 0.0;
+        double t[9];
+        auto eval = [&](auto P) {
+            constexpr bool PL = decltype(P)::value;
+            NbhRoot c;
+            const double mor3 = nbh_mor3<PL>(m, r2, c);
+            t[0] = mor3 * dx;
+            t[1] = mor3 * dy;
+            t[2] = mor3 * dz;
+            if (QUAD) {
+                const double qx = r.q0.x * dx + r.q0.y * dy + r.q1.x * dz;
+                const double qy = r.q0.y * dx + r.q1.y * dy + r.q2.x * dz;
+                const double qz = r.q1.x * dx + r.q2.x * dy + r.q2.y * dz;
+                const double dQd = qx * dx + qy * dy + qz * dz;
+                /* a body's quadrupole record is zero: its terms are too */
+                double d5 = nbh_dr5<PL>(r2, c);
+                d5 = use ? d5 : 0.0;
+                const double phiQ = nbh_phiq<PL>(d5, dQd, r2, c);
+                t[3] = phiQ * dx;
+                t[4] = phiQ * dy;
+                t[5] = phiQ * dz;
+                t[6] = -d5 * qx;
+                t[7] = -d5 * qy;
+                t[8] = -d5 * qz;
+            }
+        };
+        if (plain) eval(std::true_type()); else eval(std::false_type());
+        #pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            #pragma unroll
+            for (int k = 0; k < T; ++k) term[nbh_term_at(c, k, T, lane)] = t[c + 3 * k];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 3 * B) {
+            const int c = lane / B;                   /* lane = c * B + body */
+            double v[T][S];
+            #pragma unroll
+            for (int k = 0; k < T; ++k) {
+                const double2* from = reinterpret_cast<const double2*>(
+                    term + nbh_term_at(c, k, T, (lane % B) * S));
+                #pragma unroll
+                for (int u = 0; u < S / 2; ++u) {
+                    const double2 x = from[u];
+                    v[k][2 * u] = x.x;
+                    v[k][2 * u + 1] = x.y;
+                }
+            }
+            #pragma unroll
+            for (int u = 0; u < S; ++u) {
+                #pragma unroll
+                for (int k = 0; k < T; ++k) acc += v[k][u];
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+
+    int head = 0, tail = 0, skip = 0;                 /* skip: nothing before it is met by anyone */
+    /* the filter's nodes one chunk ahead, their indices two */
+    int q_next = lane < len ? lst[lane] : 0;
+    NodeW nd_next = node[q_next];
+    int q_after = 64 + lane < len ? lst[64 + lane] : 0;
+    for (int i0 = 0; i0 < len; i0 += 64) {
+        const bool in = i0 + lane < len;
+        const int q = q_next;
+        const NodeW nd = nd_next;
+        q_next = q_after;
+        if (i0 + 64 < len) nd_next = node[q_next];
+        q_after = i0 + 128 + lane < len ? lst[i0 + 128 + lane] : 0;
+        int opens = 0;                                /* bodies that open this node */
+        #pragma unroll
+        for (int k = 0; k < B; ++k) {
+            const double dx = nd.x - bx[k], dy = nd.y - by[k], dz = nd.z - bz[k];
+            opens += !(dz * dz + (dy * dy + dx * dx) >= nd.rcrit2);
+        }
+        if (nd.body >= 0) opens = 0;
+        const bool every = opens == 0;                /* accepted by every body */
+        /* the furthest Next of such an entry up to this lane */
+        const int reach = nbh_scan_max(in && every ? nd.next : 0);
+        const int before = max(skip, __builtin_amdgcn_update_dpp(0, reach, 0x138, 0xF, 0xF, false));
+        skip = max(skip, __builtin_amdgcn_readlane(reach, 63));
+        const bool keep = in && opens < B && q >= before;
+        const unsigned long long km = __builtin_amdgcn_ballot_w64(keep);
+        const int at = tail + (int) nbh_mbcnt(km);
+        if (keep) rnext[at & (NBH_LIST_RING - 1)] = nd.next;
+        __builtin_amdgcn_wave_barrier();
+        if (keep) {
+            unsigned cont = 0;
+            #pragma unroll
+            for (int d = 1; d < S; ++d)
+                if (rnext[(at - d) & (NBH_LIST_RING - 1)] > q) cont |= 1u << (S - d);
+            ring[at & (NBH_LIST_RING - 1)] = make_int2(q, (int) cont);
+        }
+        __builtin_amdgcn_wave_barrier();
+        tail += __popcll(km);
+        /* full batches, each one's records fetched while the one before is
+         * evaluated, in two sets of registers; the last fetch may be of stale
+         * entries, whose nodes exist */
+        int left = (tail - head) / S;
+        if (left > 0) {
+            ListRec ra = fetch(head, S);
+            for (;;) {
+                const ListRec rb = fetch(head + S, S);
+                batch(ra, S);
+                head += S;
+                if (--left == 0) break;
+                ra = fetch(head + S, S);
+                batch(rb, S);
+                head += S;
+                if (--left == 0) break;
+            }
+        }
+    }
+    if (tail > head) batch(fetch(head, tail - head), tail - head);
+
+    /* the body's three components to one lane, and whether any slot met it */
+    const unsigned long long mm = __builtin_amdgcn_ballot_w64(met);
+    if (lane < 3 * B) term[lane] = acc;
+    __builtin_amdgcn_wave_barrier();
+    const int fb = first + lane;
+    if (lane >= B || fb >= o.n) return;
+    const unsigned long long bits = (mm >> (lane * S)) & ((1ull << S) - 1ull);
+    const int fsim = simid_s[fb];
+    if (bits == 0ull) atomicOr(&sims[fsim].incest, 1u);
+    const double4 fp = spos[fb];
+    nbh_walk_finish(o, fp.x, fp.y, fp.z, term[lane], term[B + lane], term[2 * B + lane], perm[fb],
+                    oax, oay, oaz, vx, vy, vz);
+}
+
+void nbh_walk_list(nbhip_state* st, const WalkOut& o, double* oax, double* oay, double* oaz)
+{
+    hipStream_t s = st->stream;
+    const int n = st->n;
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_list_build, dim3((n + 63) / 64), dim3(NBH_LB), 0, s, st->node, st->spos,
+                       st->simid_s, st->sims, st->nkid, st->kbase, st->kid, st->wlist, st->wlen,
+                       st->scal, n, o.multi);
+#define NBH_WL(S, Q)                                                                           \
+    hipLaunchKernelGGL((k_walk_list<S, Q>), dim3((n + 64 * NBH_LW / S - 1) / (64 * NBH_LW / S)),    \
+                       dim3(64 * NBH_LW), 0,                                                   \
+                       s, st->node, st->nquad, st->spos, st->perm, st->simid_s, st->sims,      \
+                       st->wlist, st->wlen, oax, oay, oaz, st->vx, st->vy, st->vz, st->scal, o)
+    /* Four bodies a wavefront, sixteen entries a batch, while that leaves SIMDs
+     * idle: 1000 bodies 120 against 151 us (lists and walk), 4000 202 against
+     * 268, 20 000 473 against 413. */
+    if (n <= NBH_LIST_WIDE) {
+        if (st->ctx.use_quad) NBH_WL(16, true); else NBH_WL(16, false);
+    } else {
+        if (st->ctx.use_quad) NBH_WL(8, true); else NBH_WL(8, false);
+    }
+#undef NBH_WL
+}
