@@ -281,6 +281,7 @@ void nbh_masses_changed(nbhip_state* st);
 /* launchers (walk.hip) */
 void nbh_walk(nbhip_state* st, int kick, int count, double* out_ax, double* out_ay,
               double* out_az, int self_only, const WalkTune* tune);
+void nbh_list_build(nbhip_state* st);
 void nbh_walk_list(nbhip_state* st, const struct WalkOut& o, double* out_ax, double* out_ay,
                    double* out_az);
 void nbh_direct(nbhip_state* st, int nsample, const int* d_idx, double* d_acc);

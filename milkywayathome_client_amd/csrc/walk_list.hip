@@ -43,6 +43,7 @@
  * enough streaming waves to hide their chain, and the lists' LDS traffic
  * (17 LDS instructions per batch) no longer pays.
  */
+#include "nbhip_list.h"
 #include "nbhip_walk.h"
 
 #include <type_traits>
@@ -268,49 +269,6 @@ __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__
     }
 }
 
-/* Maximum over the S = 4, 8 or 16 consecutive lanes of a body. */
-template <int S>
-__device__ __forceinline__ int nbh_slots_max(int v)
-{
-    v = max(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true));              /* xor 1 */
-    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true));              /* xor 2 */
-    if (S >= 8) v = max(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true)); /* half row mirrored */
-    if (S >= 16) v = max(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true)); /* row mirrored */
-    return v;
-}
-
-/* v of one lane, uniform. */
-__device__ __forceinline__ double nbh_lane_d(double v, int lane)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int) (unsigned) (b & 0xffffffffll), lane);
-    const int hi = __builtin_amdgcn_readlane((int) (b >> 32), lane);
-    return __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-}
-
-#define NBH_LIST_RING 128
-
-/* A batch lane's node: record and quadrupole as loaded; cont has bit S - d
- * set where the entry d places back contains this one. */
-struct ListRec {
-    unsigned q, cont;
-    double2 xy, zm, rl, q0, q1, q2;
-};
-
-/* Maximum over this lane and the lanes below it. */
-__device__ __forceinline__ int nbh_scan_max(int v)
-{
-    /* row_shr 1, 2, 4, 8, then each row's last lane to the rows above
-     * (lanes without a source read 0: the values are indices >= 0) */
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false)); /* row_bcast 15 */
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false)); /* row_bcast 31 */
-    return v;
-}
-
 /* The terms in LDS: [component][term][lane], a write being one run of 64
  * doubles; the second half of the lanes two doubles on and rows of 76, which
  * keeps the adders' 16-byte reads (a body's slots, three components) on
@@ -321,148 +279,80 @@ __device__ __forceinline__ int nbh_term_at(int c, int t, int T, int lane)
     return (c * T + t) * NBH_TERM_ROW + lane + (lane >= 32 ? 2 : 0);
 }
 
-/* lane = b * S + s: body b of the wave's B = 64 / S, slot s of the batch. */
 #define NBH_LW 2                      /* wavefronts per workgroup of k_walk_list */
 template <int S, bool QUAD>
 __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restrict__ node,
-                                                   const double* __restrict__ nquad,
-                                                   const double4* __restrict__ spos,
-                                                   const unsigned* __restrict__ perm,
-                                                   const int* __restrict__ simid_s,
-                                                   SimTab* __restrict__ sims,
-                                                   const int* __restrict__ list,
-                                                   const int* __restrict__ llen,
-                                                   double* __restrict__ oax,
-                                                   double* __restrict__ oay,
-                                                   double* __restrict__ oaz,
-                                                   double* __restrict__ vx,
-                                                   double* __restrict__ vy,
-                                                   double* __restrict__ vz,
-                                                   DevScalars* __restrict__ scal, WalkOut o)
+                                                           const double* __restrict__ nquad,
+                                                           const double4* __restrict__ spos,
+                                                           const unsigned* __restrict__ perm,
+                                                           const int* __restrict__ simid_s,
+                                                           SimTab* __restrict__ sims,
+                                                           const int* __restrict__ list,
+                                                           const int* __restrict__ llen,
+                                                           double* __restrict__ oax,
+                                                           double* __restrict__ oay,
+                                                           double* __restrict__ oaz,
+                                                           double* __restrict__ vx,
+                                                           double* __restrict__ vy,
+                                                           double* __restrict__ vz,
+                                                           DevScalars* __restrict__ scal,
+                                                           WalkOut o)
 {
     constexpr int B = 64 / S;
     constexpr int T = QUAD ? 3 : 1;                   /* additions per component and entry */
-    __shared__ int2 s_ring[NBH_LW][NBH_LIST_RING];         /* pre-order index, containing entries */
+    __shared__ int2 s_ring[NBH_LW][NBH_LIST_RING];
     __shared__ int s_next[NBH_LW][NBH_LIST_RING];
     __shared__ __align__(16) double s_term[NBH_LW][3 * T * NBH_TERM_ROW];
     if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
     const int w = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
-    const int b = lane / S, slot = lane % S;
-    const int first = (blockIdx.x * NBH_LW + w) * B;       /* the wave's first body */
+    const int first = (blockIdx.x * NBH_LW + w) * B;  /* the wave's first body */
     if (first >= o.n) return;
     const int g = first >> 6;
     const int len = llen[g];
     if (len < 0) return;                              /* the streaming walk's */
-    const int* lst = list + (size_t) g * NBH_LIST_CAP;
-    int2* ring = s_ring[w];
-    int* rnext = s_next[w];
     double* term = s_term[w];
-    const int body = first + b;
-    const bool valid = body < o.n;
-    const double4 p = valid ? spos[body] : make_double4(0.0, 0.0, 0.0, 0.0);
-    /* the wave's bodies, uniform, for the filter (past the end: the first) */
-    double bx[B], by[B], bz[B];
-    {
-        const double4 f = spos[first];
-        const double vx_ = valid ? p.x : f.x, vy_ = valid ? p.y : f.y, vz_ = valid ? p.z : f.z;
-        #pragma unroll
-        for (int k = 0; k < B; ++k) {
-            bx[k] = nbh_lane_d(vx_, k * S);
-            by[k] = nbh_lane_d(vy_, k * S);
-            bz[k] = nbh_lane_d(vz_, k * S);
-        }
-    }
-    const int sim = valid ? simid_s[body] : simid_s[first];
-    const SimTab& st = sims[sim];
-    const double eps2 = st.eps2;
-    int lp = valid && st.root >= 0 ? st.root : INT_MAX;
-    const int end = o.multi ? st.end : INT_MAX;
-    const int self = valid && body < scal->nmassive ? body : -2;
-    const bool eps2_pos = o.all_eps2_pos;
-    const bool plain = __builtin_amdgcn_ballot_w64(!nbh_plain_range(st)) == 0ull;
-    bool met = false;
+    ListWave<S> L;
+    L.start(node, nquad, s_ring[w], s_next[w], first, o.n, o.multi, o.all_eps2_pos != 0, spos,
+            simid_s, sims, scal->nmassive);
     double acc = 0.0;                                 /* of body lane % B, component lane / B */
-    rnext[lane] = 0;
-    rnext[lane + 64] = 0;
-    ring[lane] = ring[lane + 64] = make_int2(0, 0);
 
-    /* entries head .. head + S - 1 of the ring */
-    auto fetch = [&](int head, int cnt) {
-        ListRec r;
-        const int2 e = ring[(head + slot) & (NBH_LIST_RING - 1)];
-        r.q = slot < cnt ? (unsigned) e.x : 0u;
-        r.cont = (unsigned) e.y;
-        /* 32-bit offsets: a state with lists has under 2^21 nodes */
-        const unsigned off = r.q * 48u;
-        const double2* rec =
-            reinterpret_cast<const double2*>(reinterpret_cast<const char*>(node) + off);
-        r.xy = rec[0];
-        r.zm = rec[1];
-        r.rl = rec[2];
-        if (QUAD) {
-            const double2* qr =
-                reinterpret_cast<const double2*>(reinterpret_cast<const char*>(nquad) + off);
-            r.q0 = qr[0];
-            r.q1 = qr[1];
-            r.q2 = qr[2];
-        }
-        return r;
-    };
-    /* one batch, `cnt` of its entries live */
-    auto batch = [&](const ListRec& r, int cnt) {
-        const bool live = slot < cnt;
-        const unsigned q = r.q;
-        const double2 xy = r.xy, zm = r.zm, rl = r.rl;
-        const long long link = __double_as_longlong(rl.y);
-        const int next = (int) (unsigned) (link & 0xffffffffll);
-        const int nbody = (int) (link >> 32);
-        const double dx = xy.x - p.x, dy = xy.y - p.y, dz = zm.x - p.z;
-        const double drSq = dz * dz + (dy * dy + dx * dx);
-        /* a node passes by itself; it is met unless it lies inside one that
-         * was accepted: before this batch (lp) or in it (cont) */
-        const bool pass = live & (drSq >= rl.x);      /* a body's rcrit2 is 0 */
-        const unsigned long long pm = __builtin_amdgcn_ballot_w64(pass);
-        const unsigned mine = (unsigned) (pm >> (b * S)) << (S - slot);
-        const bool met_here = pass & ((int) q >= lp) & ((int) q < end) & ((mine & r.cont) == 0u);
-        lp = max(lp, nbh_slots_max<S>(pass ? next : 0));
-        met |= met_here & (nbody == self);
-        const bool use = met_here & (eps2_pos | (nbody != self));
+    L.template run<QUAD>(list + (size_t) g * NBH_LIST_CAP, len, [&](const ListRec& r, int cnt) {
+        const ListHit h = L.hit(r, cnt);
         /* unused lanes: mass 0 and no quadrupole, at a harmless distance */
-        const double r2 = use ? drSq + eps2 : 1.0;
-        const double m = use ? zm.y : 0.0;
+        const double m = h.use ? r.zm.y : 0.0;
         double t[9];
         auto eval = [&](auto P) {
             constexpr bool PL = decltype(P)::value;
             NbhRoot c;
-            const double mor3 = nbh_mor3<PL>(m, r2, c);
-            t[0] = mor3 * dx;
-            t[1] = mor3 * dy;
-            t[2] = mor3 * dz;
+            const double mor3 = nbh_mor3<PL>(m, h.r2, c);
+            t[0] = mor3 * h.dx;
+            t[1] = mor3 * h.dy;
+            t[2] = mor3 * h.dz;
             if (QUAD) {
-                const double qx = r.q0.x * dx + r.q0.y * dy + r.q1.x * dz;
-                const double qy = r.q0.y * dx + r.q1.y * dy + r.q2.x * dz;
-                const double qz = r.q1.x * dx + r.q2.x * dy + r.q2.y * dz;
-                const double dQd = qx * dx + qy * dy + qz * dz;
+                const double qx = r.q0.x * h.dx + r.q0.y * h.dy + r.q1.x * h.dz;
+                const double qy = r.q0.y * h.dx + r.q1.y * h.dy + r.q2.x * h.dz;
+                const double qz = r.q1.x * h.dx + r.q2.x * h.dy + r.q2.y * h.dz;
+                const double dQd = qx * h.dx + qy * h.dy + qz * h.dz;
                 /* a body's quadrupole record is zero: its terms are too */
-                double d5 = nbh_dr5<PL>(r2, c);
-                d5 = use ? d5 : 0.0;
-                const double phiQ = nbh_phiq<PL>(d5, dQd, r2, c);
-                t[3] = phiQ * dx;
-                t[4] = phiQ * dy;
-                t[5] = phiQ * dz;
+                double d5 = nbh_dr5<PL>(h.r2, c);
+                d5 = h.use ? d5 : 0.0;
+                const double phiQ = nbh_phiq<PL>(d5, dQd, h.r2, c);
+                t[3] = phiQ * h.dx;
+                t[4] = phiQ * h.dy;
+                t[5] = phiQ * h.dz;
                 t[6] = -d5 * qx;
                 t[7] = -d5 * qy;
                 t[8] = -d5 * qz;
             }
         };
-        if (plain) eval(std::true_type()); else eval(std::false_type());
+        if (L.plain) eval(std::true_type()); else eval(std::false_type());
         #pragma unroll
         for (int c = 0; c < 3; ++c) {
             #pragma unroll
             for (int k = 0; k < T; ++k) term[nbh_term_at(c, k, T, lane)] = t[c + 3 * k];
         }
-        __builtin_amdgcn_wave_barrier();
+        nbh_wave_sync();
         if (lane < 3 * B) {
             const int c = lane / B;                   /* lane = c * B + body */
             double v[T][S];
@@ -483,71 +373,13 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
                 for (int k = 0; k < T; ++k) acc += v[k][u];
             }
         }
-        __builtin_amdgcn_wave_barrier();
-    };
-
-    int head = 0, tail = 0, skip = 0;                 /* skip: nothing before it is met by anyone */
-    /* the filter's nodes one chunk ahead, their indices two */
-    int q_next = lane < len ? lst[lane] : 0;
-    NodeW nd_next = node[q_next];
-    int q_after = 64 + lane < len ? lst[64 + lane] : 0;
-    for (int i0 = 0; i0 < len; i0 += 64) {
-        const bool in = i0 + lane < len;
-        const int q = q_next;
-        const NodeW nd = nd_next;
-        q_next = q_after;
-        if (i0 + 64 < len) nd_next = node[q_next];
-        q_after = i0 + 128 + lane < len ? lst[i0 + 128 + lane] : 0;
-        int opens = 0;                                /* bodies that open this node */
-        #pragma unroll
-        for (int k = 0; k < B; ++k) {
-            const double dx = nd.x - bx[k], dy = nd.y - by[k], dz = nd.z - bz[k];
-            opens += !(dz * dz + (dy * dy + dx * dx) >= nd.rcrit2);
-        }
-        if (nd.body >= 0) opens = 0;
-        const bool every = opens == 0;                /* accepted by every body */
-        /* the furthest Next of such an entry up to this lane */
-        const int reach = nbh_scan_max(in && every ? nd.next : 0);
-        const int before = max(skip, __builtin_amdgcn_update_dpp(0, reach, 0x138, 0xF, 0xF, false));
-        skip = max(skip, __builtin_amdgcn_readlane(reach, 63));
-        const bool keep = in && opens < B && q >= before;
-        const unsigned long long km = __builtin_amdgcn_ballot_w64(keep);
-        const int at = tail + (int) nbh_mbcnt(km);
-        if (keep) rnext[at & (NBH_LIST_RING - 1)] = nd.next;
-        __builtin_amdgcn_wave_barrier();
-        if (keep) {
-            unsigned cont = 0;
-            #pragma unroll
-            for (int d = 1; d < S; ++d)
-                if (rnext[(at - d) & (NBH_LIST_RING - 1)] > q) cont |= 1u << (S - d);
-            ring[at & (NBH_LIST_RING - 1)] = make_int2(q, (int) cont);
-        }
-        __builtin_amdgcn_wave_barrier();
-        tail += __popcll(km);
-        /* full batches, each one's records fetched while the one before is
-         * evaluated, in two sets of registers; the last fetch may be of stale
-         * entries, whose nodes exist */
-        int left = (tail - head) / S;
-        if (left > 0) {
-            ListRec ra = fetch(head, S);
-            for (;;) {
-                const ListRec rb = fetch(head + S, S);
-                batch(ra, S);
-                head += S;
-                if (--left == 0) break;
-                ra = fetch(head + S, S);
-                batch(rb, S);
-                head += S;
-                if (--left == 0) break;
-            }
-        }
-    }
-    if (tail > head) batch(fetch(head, tail - head), tail - head);
+        nbh_wave_sync();
+    });
 
     /* the body's three components to one lane, and whether any slot met it */
-    const unsigned long long mm = __builtin_amdgcn_ballot_w64(met);
+    const unsigned long long mm = __builtin_amdgcn_ballot_w64(L.met);
     if (lane < 3 * B) term[lane] = acc;
-    __builtin_amdgcn_wave_barrier();
+    nbh_wave_sync();
     const int fb = first + lane;
     if (lane >= B || fb >= o.n) return;
     const unsigned long long bits = (mm >> (lane * S)) & ((1ull << S) - 1ull);
@@ -558,14 +390,21 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
                     oax, oay, oaz, vx, vy, vz);
 }
 
+/* The groups' lists for the current tree and bodies. */
+void nbh_list_build(nbhip_state* st)
+{
+    if (st->n <= 0) return;
+    hipLaunchKernelGGL(k_list_build, dim3((st->n + 63) / 64), dim3(NBH_LB), 0, st->stream,
+                       st->node, st->spos, st->simid_s, st->sims, st->nkid, st->kbase, st->kid,
+                       st->wlist, st->wlen, st->scal, st->n, st->nsim > 1);
+}
+
 void nbh_walk_list(nbhip_state* st, const WalkOut& o, double* oax, double* oay, double* oaz)
 {
     hipStream_t s = st->stream;
     const int n = st->n;
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_list_build, dim3((n + 63) / 64), dim3(NBH_LB), 0, s, st->node, st->spos,
-                       st->simid_s, st->sims, st->nkid, st->kbase, st->kid, st->wlist, st->wlen,
-                       st->scal, n, o.multi);
+    nbh_list_build(st);
 #define NBH_WL(S, Q)                                                                           \
     hipLaunchKernelGGL((k_walk_list<S, Q>), dim3((n + 64 * NBH_LW / S - 1) / (64 * NBH_LW / S)),    \
                        dim3(64 * NBH_LW), 0,                                                   \
