@@ -366,6 +366,15 @@ __device__ __forceinline__ unsigned nbh_mbcnt(unsigned long long m)
                                      __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
 }
 
+/* LDS written by some lanes of the wave and read by others: program order is
+ * enough, kept by the compiler too. */
+__device__ __forceinline__ void nbh_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ double nbh_wave_max(double v)
 {
     for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));

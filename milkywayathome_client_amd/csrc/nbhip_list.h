@@ -31,15 +31,6 @@ __device__ __forceinline__ double nbh_lane_d(double v, int lane)
 
 #define NBH_LIST_RING 128
 
-/* LDS written by some lanes of the wave and read by others: program order is
- * enough, kept by the compiler too. */
-__device__ __forceinline__ void nbh_wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 /* A batch lane's node: record and quadrupole as loaded; cont has bit S - d
  * set where the entry d places back contains this one. */
 struct ListRec {

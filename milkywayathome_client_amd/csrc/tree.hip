@@ -1215,9 +1215,9 @@ __global__ __launch_bounds__(256) void k_level_scatter(const int* __restrict__ n
  *    go to the super-block's 64 slots.
  *  - k_sum_top: one workgroup summarises the super-blocks' spanning cells
  *    (a few per level and super-block), deepest first.
- * A cell's children come from its child list (k_fill_kids): the pre-order
- * indices of its children, sorted into octant order and checked against the
- * Next links, then loaded together instead of one after another. */
+ * One block needs no k_sum_super, one super-block no k_sum_top.
+ * A cell's children come from its child list (k_fill_kids): their pre-order
+ * indices in octant order, checked against the Next links. */
 
 /* The group walk's table (precision MIXED_GROUP): after the summaries,
  * every node's record goes to its parent's child block (slot nsim +
@@ -1295,288 +1295,313 @@ struct SumView {
     int nn;
 };
 
-#define NBH_NO_KID 0x7fffffff   /* an unused slot of a sorted child list */
-#define NBH_KID_CELL 0x80000000u /* flag of a child list entry: the child is a cell */
-
-/* The structure half of a cell's summary: its children, sorted into
- * pre-order (= octant order), into ch[8] (unused slots NBH_NO_KID; cells
- * flagged NBH_KID_CELL), checked against the Next links; false on a child
- * list that disagrees with them (a corrupt table).  Reads structure only
- * (levels, Next links, child lists), so it may run before the children are
- * summarised. */
-__device__ __forceinline__ bool nbh_cell_children(const SumView& v, int p, int* __restrict__ out)
-{
-    /* without branches (a failed check clears ok and later loads use safe
-     * indices), so that two inlined calls overlap their three rounds of
-     * dependent loads */
-    const int level = v.nlevel[p];
-    const int end = v.nnext[p];
-    const int nk = __popc(v.g.nkid[p]);
-    const int kbr = (int) v.g.kbase[p];
-    bool ok = !(level < 0 || end <= p + 1 || end > v.nn || nk < 1 || nk > 8);
-    const int kb = ok ? kbr : 0;
-    int ch[8];
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) ch[j] = (ok && j < nk) ? v.kid[kb + j] : NBH_NO_KID;
-    /* Batcher's odd-even merge network for 8 keys (19 compare-exchanges,
-     * static indices: the list stays in registers) */
-#define NBH_CE(a, b)                                                    \
-    do {                                                                \
-        const int lo_ = min(ch[a], ch[b]), hi_ = max(ch[a], ch[b]);     \
-        ch[a] = lo_;                                                    \
-        ch[b] = hi_;                                                    \
-    } while (0)
-    NBH_CE(0, 1); NBH_CE(2, 3); NBH_CE(4, 5); NBH_CE(6, 7);
-    NBH_CE(0, 2); NBH_CE(1, 3); NBH_CE(4, 6); NBH_CE(5, 7);
-    NBH_CE(1, 2); NBH_CE(5, 6);
-    NBH_CE(0, 4); NBH_CE(1, 5); NBH_CE(2, 6); NBH_CE(3, 7);
-    NBH_CE(2, 4); NBH_CE(3, 5);
-    NBH_CE(1, 2); NBH_CE(3, 4); NBH_CE(5, 6);
-#undef NBH_CE
-    ok = ok && ch[0] == p + 1;
-    #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        if (j < nk) ok = ok && ch[j] >= 0 && ch[j] < v.nn;
-    int lv[8], nx[8];
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const bool use = ok && j < nk;
-        const int c = use ? ch[j] : 0;
-        lv[j] = use ? v.nlevel[c] : -1;
-        const int nn = use ? v.nnext[c] : 0;
-        nx[j] = use ? (lv[j] < 0 ? ch[j] + 1 : nn) : 0;
-    }
-    /* the list must be the Next chain p+1 -> ... -> end */
-    #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        if (j < nk) ok = ok && nx[j] == (j + 1 < nk ? ch[j + 1] : end);
-    #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        out[j] = j < nk ? (int) ((unsigned) ch[j] | (lv[j] >= 0 ? NBH_KID_CELL : 0u)) : NBH_NO_KID;
-    return ok;
-}
-
-/* The value half: the cell's record (centre of mass, mass, critical
- * radius, quadrupole, and the mixed walk's record) from its children's
- * finished records; chl is the cell's checked, sorted, flagged child list.
- * The children's positions and masses and the quadrupoles of the child
- * cells are loaded together (the flags say which children are cells). */
-__device__ __forceinline__ void nbh_cell_summary(const SumView& v, int p, const int* __restrict__ chl)
-{
-    NodeW* __restrict__ node = v.node;
-    int ch[8];
-    bool cell[8];
-    int nk = 0;
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int e = chl[j];
-        nk += e != NBH_NO_KID;
-        cell[j] = e != NBH_NO_KID && ((unsigned) e & NBH_KID_CELL);
-        ch[j] = e & 0x7fffffff;
-    }
-    const int level = v.nlevel[p];
-    const int sim = v.nsim[p];
-    const double rsize = v.sims[sim].rsize;
-    const int end = v.nnext[p];
-    const bool quad = v.ctx.use_quad != 0;
-    double4 w[8];                                  /* x y z m */
-    double cq[8][6];
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        if (j < nk) w[j] = *reinterpret_cast<const double4*>(&node[ch[j]]);
-        #pragma unroll
-        for (int k = 0; k < 6; ++k)
-            cq[j][k] = (quad && j < nk && cell[j]) ? v.nquad[6 * (size_t) ch[j] + k] : 0.0;
-    }
-
-    double mass = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        if (j < nk) {
-            mass += w[j].w;
-            cx += w[j].w * w[j].x;
-            cy += w[j].w * w[j].y;
-            cz += w[j].w * w[j].z;
-        }
-    }
-    const double mx = v.nmid[3 * p + 0], my = v.nmid[3 * p + 1], mz = v.nmid[3 * p + 2];
-    if (mass > 0.0) {
-        cx /= mass;
-        cy /= mass;
-        cz /= mass;
-    } else {
-        cx = mx; cy = my; cz = mz;
-    }
-    const double psize = ldexp(rsize, -level);
-    const double half = 0.5 * psize;
-    if (cx < mx - half || cx > mx + half || cy < my - half || cy > my + half ||
-        cz < mz - half || cz > mz + half)
-        atomicOr(&v.sims[sim].flags, NBHIP_TREE_STRUCTURE_ERROR);
-    const double rc2 = nbh_rcrit2(v.ctx, mx, my, mz, rsize, cx, cy, cz, psize);
-
-    double* pq = &v.nquad[6 * (size_t) p];
-    if (quad) {
-        double q0 = 0.0, q1 = 0.0, q2 = 0.0, q3 = 0.0, q4 = 0.0, q5 = 0.0;
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (j >= nk) continue;
-            const double dx = w[j].x - cx, dy = w[j].y - cy, dz = w[j].z - cz;
-            const double drsq = dz * dz + (dy * dy + dx * dx);
-            const double m = w[j].w;
-            double e0 = m * (3.0 * (dx * dx) - drsq);
-            double e1 = m * (3.0 * (dx * dy));
-            double e2 = m * (3.0 * (dx * dz));
-            double e3 = m * (3.0 * (dy * dy) - drsq);
-            double e4 = m * (3.0 * (dy * dz));
-            double e5 = m * (3.0 * (dz * dz) - drsq);
-            if (cell[j]) {
-                e0 += cq[j][0]; e1 += cq[j][1]; e2 += cq[j][2];
-                e3 += cq[j][3]; e4 += cq[j][4]; e5 += cq[j][5];
-            }
-            q0 += e0; q1 += e1; q2 += e2; q3 += e3; q4 += e4; q5 += e5;
-        }
-        pq[0] = q0; pq[1] = q1; pq[2] = q2; pq[3] = q3; pq[4] = q4; pq[5] = q5;
-        if (v.nodef) {
-            NodeF& f = v.nodef[p];
-            f.q[0] = (float) q0; f.q[1] = (float) q1; f.q[2] = (float) q2;
-            f.q[3] = (float) q3; f.q[4] = (float) q4; f.q[5] = (float) q5;
-        }
-    } else {
-        pq[0] = pq[1] = pq[2] = pq[3] = pq[4] = pq[5] = 0.0;
-        if (v.nodef)
-            for (int k = 0; k < 6; ++k) v.nodef[p].q[k] = 0.0f;
-    }
-    NodeW r;
-    r.x = cx;
-    r.y = cy;
-    r.z = cz;
-    r.m = mass;
-    r.rcrit2 = rc2;
-    r.next = end;
-    r.body = -1;
-    node[p] = r;
-    if (v.nodef) {
-        /* the mixed walk's record: FP64 position, the rest in FP32 */
-        NodeF& f = v.nodef[p];
-        f.x = cx;
-        f.y = cy;
-        f.z = cz;
-        f.m = (float) mass;
-        /* the coherent walk may open more (rc_scale >= 1; 1 otherwise) */
-        f.rcrit2 = (float) (rc2 * v.rc_scale);
-        f.next = end;
-        f.body = -1;
-    }
-}
-
-/* One cell's summary; false on a child list that disagrees with the Next
- * links (a corrupt table). */
-__device__ __forceinline__ bool nbh_summarize_cell(const SumView& v, int p)
-{
-    int ch[8];
-    if (!nbh_cell_children(v, p, ch)) return false;
-    nbh_cell_summary(v, p, ch);
-    return true;
-}
-
-#define NBH_SUM_BODIES 1024    /* massive bodies per k_sum_blocks workgroup */
-#define NBH_SUM_THREADS 256
-#define NBH_SUMB_THREADS 128   /* k_sum_blocks: two waves, so that with its ~220 VGPRs
-                                  four workgroups share a CU and all blocks of a
-                                  10^6-body tree run at once */
-#define NBH_SUM_GROUP 64       /* blocks per k_sum_super workgroup */
+/* A pass costs its launch, its chain of dependent reads and its levels; the
+ * blocks are small because those come once per launch while the cells of a
+ * block come one round of NBH_SUMB_THREADS/8 after the other.  192 bodies a
+ * block: 20 us (10^3 bodies), the next pass 42 (2x10^4), 129 (10^6, blocks
+ * alone); 256: 21, 35, 125; 384: 26, 31, 123; 512: 33, 30, 144. */
+#define NBH_SUM_BODIES 256     /* massive bodies per k_sum_blocks workgroup */
+#define NBH_SUMB_THREADS 256
+#define NBH_SUMB_REG 8         /* table entries per thread held in registers */
+/* Cells whose records a workgroup keeps in LDS.  256 bodies have about 140
+ * cells, more where bodies cluster; 256 instead of 320 sends enough blocks of
+ * a 10^6-body Plummer sphere past the limit to take 165 us instead of 125. */
+#define NBH_SUMB_KEEP 320
+/* Blocks per k_sum_super workgroup: 128 summarise 32768 bodies, so that
+ * states up to that size need no k_sum_top (18 us at 2x10^4 bodies with 64,
+ * against 6 us more here). */
+#define NBH_SUM_GROUP 128
+#define NBH_SUM_THREADS 512    /* k_sum_super, k_sum_top */
+#define NBH_SUM_KEEP 512       /* NBH_SUMB_KEEP of k_sum_super */
+#define NBH_SUMT_KEEP 1024     /* and of k_sum_top (10^6 bodies: about 600 cells) */
 #define NBH_SPAN_SLOTS 64      /* spanning cells one block can hand up (one per level) */
-#define NBH_SPAN_THREADS 512
-#define NBH_SUM_CAP 1024       /* cells whose child lists a workgroup keeps in LDS */
-#define NBH_SUMB_REG 16        /* k_sum_blocks: table entries per thread held in registers */
+/* Cells of a team read ahead together: k_sum_blocks has its other waves to
+ * wait for (1: 125 us at 10^6 bodies, 2: 153), the others do not
+ * (4: 17.8 us at 10^3 bodies, 2: 14.9). */
+#define NBH_SUMB_ROUNDS 1
+#define NBH_SUM_ROUNDS 2
 
-/* off[l] = cells of levels < l, off[64] = all (exclusive scan of the 64
- * level counts cnt[], by the first wave; callers synchronise after) */
-__device__ __forceinline__ void nbh_level_offsets(const int* cnt, int* off)
+/* A finished cell as its parent needs it: x y z m, then the quadrupole. */
+struct CellRec {
+    double d[10];
+};
+
+/* A team of 8 lanes' terms: one row of 8 children per sum. */
+#define NBH_SUM_TERMS 50       /* doubles per team: 6 rows and 2 to spread the banks */
+
+/* The levels of a workgroup's cells: off[l] = cells of levels < l, off[64] =
+ * all, used has a bit per level that holds any. */
+struct SumLevels {
+    int cnt[64];
+    int off[65];
+    int fill[64];
+    unsigned long long used;
+};
+
+/* Offsets and used levels from the counts, by the first wave; callers
+ * synchronise after. */
+__device__ __forceinline__ void nbh_level_offsets(SumLevels& lv)
 {
     if (threadIdx.x < 64) {
-        const int c = cnt[threadIdx.x];
+        const int c = lv.cnt[threadIdx.x];
         int x = c;
         for (int o = 1; o < 64; o <<= 1) {
             const int y = __shfl_up(x, o, 64);
             if ((int) threadIdx.x >= o) x += y;
         }
-        off[threadIdx.x] = x - c;
-        if (threadIdx.x == 63) off[64] = x;
+        lv.off[threadIdx.x] = x - c;
+        if (threadIdx.x == 63) lv.off[64] = x;
+        const unsigned long long used = __ballot(c > 0);
+        if (threadIdx.x == 0) lv.used = used;
     }
 }
 
-/* Summaries of the cells list[0 .. off[64]), grouped by level (level l at
- * list[off[l] .. off[l+1])), deepest level first, one barrier per level.
- * Up to NBH_SUM_CAP cells, every cell's child list is read, sorted and
- * checked first, all levels at once, and kept in LDS (s_ch: two int4 per
- * cell), so that a level then waits on one round of loads -- its children's
- * records -- instead of the chain nlevel/kbase -> kid -> children.  More
- * cells: each level does both halves.  False on a corrupt child list. */
-template <int NT>
-__device__ bool nbh_sum_levels(const SumView& v, const int* list, const int* off, int4* s_ch)
+/* A cell as lane e of its team holds it: the cell's place, and child e. */
+struct TeamCell {
+    int p, at, level, end, sim, nk;
+    int ch, from;                 /* child e; its list place if it is a cell of this pass, or -1 */
+    bool cell;
+    double rsize, mx, my, mz;
+    double4 w;                    /* child e: x y z m, zeros past the last child */
+    double q[6];                  /* and its quadrupole if it is a cell */
+};
+
+/* Summaries of the cells list[0 .. lv.off[64]), grouped by level (level l at
+ * list[off[l] .. off[l+1])), deepest level first: centre of mass, mass,
+ * critical radius, quadrupole, and the mixed walk's record.
+ *
+ * A pass is a serial chain of levels: what bounds it is one level's time, not
+ * the work.  A team of 8 lanes takes a cell, lane e its child e: the products
+ * of all children at once, then lane k adds term k of the children in their
+ * order (exchanged through LDS).  R cells of a team are read ahead together,
+ * children that are final already (bodies, cells of earlier launches) with
+ * their records; a level then waits for the records that deeper levels of
+ * this pass left in LDS (rec, if keep), not for stores to reach the table and
+ * come back.  With more cells than rec holds (!keep) a level reads its
+ * children from the table, after a full barrier.  Three launches together,
+ * with a thread per cell (and its children one after the other), then now:
+ * 126 and 36 us (10^3 bodies), 120 and 54 (2x10^4), 259 and 212 (10^6).
+ *
+ * The child lists are checked against the Next links: children must be the
+ * chain p+1 -> ... -> Next of p.  False on a list that is not (a corrupt
+ * table); the status that it sets stops the step.  slot(q): the list place
+ * of cell q if it is one of these cells, any number otherwise (checked
+ * against the list). */
+template <int NT, int R, class Slot>
+__device__ bool nbh_sum_cells(const SumView& v, const int* list, const SumLevels& lv, bool keep,
+                              CellRec* rec, double* terms, Slot&& slot)
 {
-    const int tid = threadIdx.x;
-    const int total = off[64];
-    bool ok = true;
-    if (total <= NBH_SUM_CAP) {
-        /* two cells per round, their loads overlapped */
-        auto keep = [&](int i, bool good, const int* ch) {
-            if (good) {
-                s_ch[2 * i] = make_int4(ch[0], ch[1], ch[2], ch[3]);
-                s_ch[2 * i + 1] = make_int4(ch[4], ch[5], ch[6], ch[7]);
-            } else {
-                ok = false;                               /* marked: a list never starts empty */
-                s_ch[2 * i] = make_int4(NBH_NO_KID, NBH_NO_KID, NBH_NO_KID, NBH_NO_KID);
-            }
-        };
-        for (int i = tid; i < total; i += 2 * NT) {
-            const int i1 = i + NT;
-            const bool has1 = i1 < total;
-            int c0[8], c1[8];
-            const bool g0 = nbh_cell_children(v, list[i], c0);
-            const bool g1 = nbh_cell_children(v, list[has1 ? i1 : i], c1);
-            keep(i, g0, c0);
-            if (has1) keep(i1, g1, c1);
+    constexpr int T = NT / 8;
+    const int tid = threadIdx.x, e = tid & 7, team = tid >> 3;
+    double* const t = terms + team * NBH_SUM_TERMS;
+    const bool quad = v.ctx.use_quad != 0;
+    const int total = lv.off[64];
+    unsigned long long left = lv.used;
+    bool good = true;
+    for (int base = 0; base < total; base += R * T) {
+        TeamCell c[R];
+        /* four rounds of dependent loads, R cells in each */
+        int kb[R];
+        #pragma unroll
+        for (int r = 0; r < R; ++r) {
+            c[r].at = total - 1 - (base + r * T + team);
+            c[r].p = c[r].at >= 0 ? list[c[r].at] : -1;
         }
-        __syncthreads();
-        for (int l = 63; l >= 0; --l) {
-            if (off[l + 1] == off[l]) continue;           /* uniform */
-            for (int i = off[l] + tid; i < off[l + 1]; i += NT) {
-                const int4 a = s_ch[2 * i];
-                if (a.x == NBH_NO_KID) continue;
-                const int4 b = s_ch[2 * i + 1];
-                const int ch[8] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w };
-                nbh_cell_summary(v, list[i], ch);
-            }
-            __syncthreads();
+        #pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool has = c[r].p >= 0;
+            const int p = has ? c[r].p : 0;
+            c[r].level = has ? v.nlevel[p] : -1;
+            c[r].end = v.nnext[p];
+            c[r].sim = v.nsim[p];
+            c[r].nk = __popc(v.g.nkid[p]);
+            kb[r] = (int) v.g.kbase[p];
+            c[r].mx = v.nmid[3 * p + 0];
+            c[r].my = v.nmid[3 * p + 1];
+            c[r].mz = v.nmid[3 * p + 2];
         }
-    } else {
-        for (int l = 63; l >= 0; --l) {
-            if (off[l + 1] == off[l]) continue;           /* uniform */
-            for (int i = off[l] + tid; i < off[l + 1]; i += NT)
-                ok = nbh_summarize_cell(v, list[i]) && ok;
-            __syncthreads();
+        #pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool ok = c[r].level >= 0 && c[r].end > c[r].p + 1 && c[r].end <= v.nn &&
+                            c[r].nk >= 1 && c[r].nk <= 8;
+            if (c[r].p >= 0 && !ok) good = false;
+            if (!ok) c[r].level = -1;
+            c[r].ch = ok && e < c[r].nk ? v.kid[kb[r] + e] : -1;
+            c[r].rsize = ok ? v.sims[c[r].sim].rsize : 0.0;
+        }
+        #pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool use = c[r].level >= 0 && e < c[r].nk;
+            const bool in = use && c[r].ch >= 0 && c[r].ch < v.nn;
+            const int q = in ? c[r].ch : 0;
+            const int ql = v.nlevel[q];
+            const int qn = ql < 0 ? q + 1 : v.nnext[q];
+            c[r].cell = in && ql >= 0;
+            const int after = __shfl_down(c[r].ch, 1, 8);
+            bool ok = !use || (in && qn == (e + 1 < c[r].nk ? after : c[r].end));
+            if (use && e == 0) ok = ok && c[r].ch == c[r].p + 1;
+            /* the verdict of the team's eight lanes */
+            if ((__ballot(ok) >> (tid & 56) & 0xffull) != 0xffull) {
+                good = false;
+                c[r].level = -1;
+            }
+            int f = c[r].cell ? slot(q) : -1;
+            if (f < 0 || f >= total || list[f] != q) f = -1;
+            c[r].from = f;
+            c[r].w = make_double4(0.0, 0.0, 0.0, 0.0);
+            #pragma unroll
+            for (int k = 0; k < 6; ++k) c[r].q[k] = 0.0;
+            if (keep && in && f < 0) {
+                c[r].w = *reinterpret_cast<const double4*>(&v.node[q]);
+                if (quad && c[r].cell) {
+                    #pragma unroll
+                    for (int k = 0; k < 6; ++k) c[r].q[k] = v.nquad[6 * (size_t) q + k];
+                }
+            }
+        }
+        #pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int lo = total - (base + (r + 1) * T);   /* the round's places: [lo, lo + T) */
+            while (left) {                                 /* uniform */
+                const int l = 63 - __clzll((long long) left);
+                if (lv.off[l + 1] <= lo) break;
+                if (c[r].level == l) {
+                    const TeamCell& s = c[r];
+                    double4 w = s.w;
+                    double cq[6];
+                    #pragma unroll
+                    for (int k = 0; k < 6; ++k) cq[k] = s.q[k];
+                    if (keep && s.from >= 0) {
+                        const CellRec& k = rec[s.from];
+                        w = make_double4(k.d[0], k.d[1], k.d[2], k.d[3]);
+                        #pragma unroll
+                        for (int j = 0; j < 6; ++j) cq[j] = k.d[4 + j];
+                    } else if (!keep && e < s.nk) {
+                        w = *reinterpret_cast<const double4*>(&v.node[s.ch]);
+                        if (quad && s.cell) {
+                            #pragma unroll
+                            for (int k = 0; k < 6; ++k) cq[k] = v.nquad[6 * (size_t) s.ch + k];
+                        }
+                    }
+                    t[0 + e] = w.w;
+                    t[8 + e] = w.w * w.x;
+                    t[16 + e] = w.w * w.y;
+                    t[24 + e] = w.w * w.z;
+                    nbh_wave_sync();
+                    /* zeros past the last child change no sum: a sum that
+                     * began at +0 is never -0 */
+                    double mass = 0.0, sum = 0.0;
+                    #pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        mass += t[j];
+                        sum += t[8 * (e & 3) + j];
+                    }
+                    nbh_wave_sync();
+                    double cx = s.mx, cy = s.my, cz = s.mz;
+                    if (mass > 0.0) {
+                        const double cen = sum / mass;
+                        cx = __shfl(cen, 1, 8);
+                        cy = __shfl(cen, 2, 8);
+                        cz = __shfl(cen, 3, 8);
+                    }
+                    const double psize = ldexp(s.rsize, -s.level);
+                    const double half = 0.5 * psize;
+                    if (e == 0 && (cx < s.mx - half || cx > s.mx + half || cy < s.my - half ||
+                                   cy > s.my + half || cz < s.mz - half || cz > s.mz + half))
+                        atomicOr(&v.sims[s.sim].flags, NBHIP_TREE_STRUCTURE_ERROR);
+                    const double rc2 =
+                        nbh_rcrit2(v.ctx, s.mx, s.my, s.mz, s.rsize, cx, cy, cz, psize);
+                    double qk = 0.0;                       /* lane k < 6: quadrupole term k */
+                    if (quad) {
+                        const double dx = w.x - cx, dy = w.y - cy, dz = w.z - cz;
+                        const double drsq = dz * dz + (dy * dy + dx * dx);
+                        const double m = w.w;
+                        double e0 = m * (3.0 * (dx * dx) - drsq);
+                        double e1 = m * (3.0 * (dx * dy));
+                        double e2 = m * (3.0 * (dx * dz));
+                        double e3 = m * (3.0 * (dy * dy) - drsq);
+                        double e4 = m * (3.0 * (dy * dz));
+                        double e5 = m * (3.0 * (dz * dz) - drsq);
+                        if (s.cell) {
+                            e0 += cq[0]; e1 += cq[1]; e2 += cq[2];
+                            e3 += cq[3]; e4 += cq[4]; e5 += cq[5];
+                        }
+                        const bool use = e < s.nk;
+                        t[0 + e] = use ? e0 : 0.0;
+                        t[8 + e] = use ? e1 : 0.0;
+                        t[16 + e] = use ? e2 : 0.0;
+                        t[24 + e] = use ? e3 : 0.0;
+                        t[32 + e] = use ? e4 : 0.0;
+                        t[40 + e] = use ? e5 : 0.0;
+                        nbh_wave_sync();
+                        const int row = 8 * (e < 6 ? e : 5);
+                        #pragma unroll
+                        for (int j = 0; j < 8; ++j) qk += t[row + j];
+                        nbh_wave_sync();
+                    }
+                    if (keep) {
+                        CellRec& k = rec[s.at];
+                        if (e < 4) k.d[e] = e == 0 ? cx : e == 1 ? cy : e == 2 ? cz : mass;
+                        if (e < 6) k.d[4 + e] = qk;
+                    }
+                    if (e < 6) {
+                        v.nquad[6 * (size_t) s.p + e] = qk;
+                        if (v.nodef) v.nodef[s.p].q[e] = (float) qk;
+                    }
+                    if (e == 0) {
+                        NodeW o;
+                        o.x = cx;
+                        o.y = cy;
+                        o.z = cz;
+                        o.m = mass;
+                        o.rcrit2 = rc2;
+                        o.next = s.end;
+                        o.body = -1;
+                        v.node[s.p] = o;
+                        if (v.nodef) {
+                            /* the mixed walk's record: FP64 position, the rest in FP32 */
+                            NodeF& f = v.nodef[s.p];
+                            f.x = cx;
+                            f.y = cy;
+                            f.z = cz;
+                            f.m = (float) mass;
+                            /* the coherent walk may open more (rc_scale >= 1; 1 otherwise) */
+                            f.rcrit2 = (float) (rc2 * v.rc_scale);
+                            f.next = s.end;
+                            f.body = -1;
+                        }
+                    }
+                }
+                if (keep) {
+                    /* the level's records are in LDS; nobody in this launch
+                     * waits for its stores to the table */
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                } else {
+                    __syncthreads();
+                }
+                if (lv.off[l] < lo) break;                 /* the level goes on in the next round */
+                left &= ~(1ull << l);
+            }
         }
     }
-    return ok;
+    return good;
 }
 
-/* Levels holding cells in [lo, hi): counts into cnt[64] (LDS), then an
- * exclusive scan into off[65]; callers add their own cells. */
-__global__ __launch_bounds__(NBH_SUMB_THREADS) void k_sum_blocks(SumView v,
+__global__ __launch_bounds__(NBH_SUMB_THREADS, 3) void k_sum_blocks(SumView v,
                                                                 const unsigned* __restrict__ cincl,
                                                                 int* __restrict__ blist,
                                                                 int* __restrict__ span,
                                                                 int* __restrict__ span_n,
                                                                 DevScalars* __restrict__ scal)
 {
-    __shared__ int cnt[64];
-    __shared__ int off[65];
-    __shared__ int fill[64];
+    __shared__ SumLevels lv;
     __shared__ int nspan;
-    __shared__ int s_list[NBH_SUM_CAP];
-    __shared__ int4 s_ch[2 * NBH_SUM_CAP];
+    __shared__ int s_list[NBH_SUMB_KEEP];
+    __shared__ unsigned short s_slot[NBH_SUMB_REG * NBH_SUMB_THREADS];
+    __shared__ CellRec rec[NBH_SUMB_KEEP];
+    __shared__ double terms[NBH_SUMB_THREADS / 8 * NBH_SUM_TERMS];
     const int tid = threadIdx.x;
     if (scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) return;
     const int M = scal->nmassive;
@@ -1586,8 +1611,8 @@ __global__ __launch_bounds__(NBH_SUMB_THREADS) void k_sum_blocks(SumView v,
     const int P0 = b0 + (b0 > 0 ? (int) cincl[b0 - 1] : 0);
     const int P1 = min((b1 - 1) + (int) cincl[b1 - 1] + 1, v.nn);
     if (tid < 64) {
-        cnt[tid] = 0;
-        fill[tid] = 0;
+        lv.cnt[tid] = 0;
+        lv.fill[tid] = 0;
     }
     if (tid == 0) nspan = 0;
     __syncthreads();
@@ -1611,7 +1636,7 @@ __global__ __launch_bounds__(NBH_SUMB_THREADS) void k_sum_blocks(SumView v,
             return;
         }
         if (nx <= P1) {
-            atomicAdd(&cnt[l], 1);
+            atomicAdd(&lv.cnt[l], 1);
         } else {
             const int k = atomicAdd(&nspan, 1);
             if (k < NBH_SPAN_SLOTS)
@@ -1628,15 +1653,18 @@ __global__ __launch_bounds__(NBH_SUMB_THREADS) void k_sum_blocks(SumView v,
     }
     __syncthreads();
     if (tid == 0) span_n[blockIdx.x] = min(nspan, NBH_SPAN_SLOTS);
-    nbh_level_offsets(cnt, off);
+    nbh_level_offsets(lv);
     __syncthreads();
     /* the block's inside cells grouped by level: in LDS, or, past
-     * NBH_SUM_CAP, in the block's own slice [P0, P0 + count) of blist
+     * NBH_SUMB_KEEP, in the block's own slice [P0, P0 + count) of blist
      * (slices of different blocks are disjoint) */
-    int* lst = off[64] <= NBH_SUM_CAP ? s_list : blist + P0;
+    int* lst = lv.off[64] <= NBH_SUMB_KEEP ? s_list : blist + P0;
     auto place = [&](int q, int l, int nx) {
+        if (in_regs && q < P1) s_slot[q - P0] = 0xffff;
         if (l < 0 || l > 63 || nx > P1) return;
-        lst[off[l] + atomicAdd(&fill[l], 1)] = q;
+        const int i = lv.off[l] + atomicAdd(&lv.fill[l], 1);
+        lst[i] = q;
+        if (in_regs) s_slot[q - P0] = (unsigned short) i;
     };
     if (in_regs) {
         #pragma unroll
@@ -1645,22 +1673,26 @@ __global__ __launch_bounds__(NBH_SUMB_THREADS) void k_sum_blocks(SumView v,
         for (int q = P0 + tid; q < P1; q += NBH_SUMB_THREADS) place(q, v.nlevel[q], v.nnext[q]);
     }
     __syncthreads();
-    if (!nbh_sum_levels<NBH_SUMB_THREADS>(v, lst, off, s_ch)) atomicOr(&scal->status, NBHIP_ERROR);
+    const bool keep = in_regs && lv.off[64] <= NBH_SUMB_KEEP;
+    if (!nbh_sum_cells<NBH_SUMB_THREADS, NBH_SUMB_ROUNDS>(v, lst, lv, keep, rec, terms, [&](int q) {
+            return keep && q >= P0 && q < P1 ? (int) s_slot[q - P0] : -1;
+        }))
+        atomicOr(&scal->status, NBHIP_ERROR);
 }
 
 /* Cells handed up by several lower workgroups (cand[0..nc) in LDS or
  * global memory), grouped by level in LDS and summarised deepest level
  * first; those whose subtree ends past P1 go to out[0..NBH_SPAN_SLOTS)
  * instead (out may be null when P1 covers the whole table). */
-template <int NT>
+template <int NT, int KEEP>
 __device__ void nbh_sum_handed(const SumView& v, const int* cand, int nc, int P1, int* out,
-                               int* out_n, int* list, int* cnt, int* off, int* fill, int* nspan,
-                               int4* s_ch, DevScalars* scal)
+                               int* out_n, int* list, SumLevels& lv, int* nspan, CellRec* rec,
+                               double* terms, int* slot, DevScalars* scal)
 {
     const int tid = threadIdx.x;
     if (tid < 64) {
-        cnt[tid] = 0;
-        fill[tid] = 0;
+        lv.cnt[tid] = 0;
+        lv.fill[tid] = 0;
     }
     if (tid == 0) *nspan = 0;
     __syncthreads();
@@ -1672,7 +1704,7 @@ __device__ void nbh_sum_handed(const SumView& v, const int* cand, int nc, int P1
             continue;
         }
         if (v.nnext[q] <= P1) {
-            atomicAdd(&cnt[l], 1);
+            atomicAdd(&lv.cnt[l], 1);
         } else {
             const int k = atomicAdd(nspan, 1);
             if (out && k < NBH_SPAN_SLOTS) out[k] = q;
@@ -1680,17 +1712,21 @@ __device__ void nbh_sum_handed(const SumView& v, const int* cand, int nc, int P1
         }
     }
     __syncthreads();
-    nbh_level_offsets(cnt, off);
+    nbh_level_offsets(lv);
     if (tid == 0 && out_n) *out_n = min(*nspan, NBH_SPAN_SLOTS);
     __syncthreads();
     for (int i = tid; i < nc; i += NT) {
         const int q = cand[i];
         const int l = v.nlevel[q];
         if (l < 0 || l > 63 || v.nnext[q] > P1) continue;
-        list[off[l] + atomicAdd(&fill[l], 1)] = q;
+        const int at = lv.off[l] + atomicAdd(&lv.fill[l], 1);
+        list[at] = q;
+        slot[q] = at;
     }
     __syncthreads();
-    if (!nbh_sum_levels<NT>(v, list, off, s_ch)) atomicOr(&scal->status, NBHIP_ERROR);
+    if (!nbh_sum_cells<NT, NBH_SUM_ROUNDS>(v, list, lv, lv.off[64] <= KEEP, rec, terms,
+                           [&](int q) { return slot[q]; }))
+        atomicOr(&scal->status, NBHIP_ERROR);
 }
 
 /* Workgroup s: the spanning cells of blocks [s*NBH_SUM_GROUP, ...). */
@@ -1700,16 +1736,16 @@ __global__ __launch_bounds__(NBH_SUM_THREADS) void k_sum_super(SumView v,
                                                                const int* __restrict__ span_n,
                                                                int* __restrict__ span2,
                                                                int* __restrict__ span2_n,
+                                                               int* slot,
                                                                DevScalars* __restrict__ scal)
 {
     __shared__ int cand[NBH_SUM_GROUP * NBH_SPAN_SLOTS];
     __shared__ int list[NBH_SUM_GROUP * NBH_SPAN_SLOTS];
-    __shared__ int cnt[64];
-    __shared__ int off[65];
-    __shared__ int fill[64];
+    __shared__ SumLevels lv;
     __shared__ int nspan;
     __shared__ int ncand;
-    __shared__ int4 s_ch[2 * NBH_SUM_CAP];
+    __shared__ CellRec rec[NBH_SUM_KEEP];
+    __shared__ double terms[NBH_SUM_THREADS / 8 * NBH_SUM_TERMS];
     const int tid = threadIdx.x;
     if (scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) return;
     const int M = scal->nmassive;
@@ -1727,25 +1763,24 @@ __global__ __launch_bounds__(NBH_SUM_THREADS) void k_sum_super(SumView v,
         for (int j = 0; j < c; ++j) cand[base + j] = span[(size_t) k * NBH_SPAN_SLOTS + j];
     }
     __syncthreads();
-    nbh_sum_handed<NBH_SUM_THREADS>(v, cand, ncand, P1, span2 + (size_t) blockIdx.x * NBH_SPAN_SLOTS,
-                                    span2_n + blockIdx.x, list, cnt, off, fill, &nspan, s_ch,
-                                    scal);
+    nbh_sum_handed<NBH_SUM_THREADS, NBH_SUM_KEEP>(v, cand, ncand, P1, span2 + (size_t) blockIdx.x * NBH_SPAN_SLOTS,
+                                    span2_n + blockIdx.x, list, lv, &nspan, rec, terms,
+                                    slot, scal);
 }
 
 /* One workgroup: every super-block's spanning cells. */
-__global__ __launch_bounds__(NBH_SPAN_THREADS) void k_sum_top(SumView v,
+__global__ __launch_bounds__(NBH_SUM_THREADS) void k_sum_top(SumView v,
                                                               const int* __restrict__ span2,
                                                               const int* __restrict__ span2_n,
                                                               int nsuper, int* __restrict__ cand,
-                                                              int* __restrict__ list,
+                                                              int* list, int* slot,
                                                               DevScalars* __restrict__ scal)
 {
-    __shared__ int cnt[64];
-    __shared__ int off[65];
-    __shared__ int fill[64];
+    __shared__ SumLevels lv;
     __shared__ int nspan;
     __shared__ int ncand;
-    __shared__ int4 s_ch[2 * NBH_SUM_CAP];
+    __shared__ CellRec rec[NBH_SUMT_KEEP];
+    __shared__ double terms[NBH_SUM_THREADS / 8 * NBH_SUM_TERMS];
     const int tid = threadIdx.x;
     if (scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) return;
     const int M = scal->nmassive;
@@ -1753,14 +1788,14 @@ __global__ __launch_bounds__(NBH_SPAN_THREADS) void k_sum_top(SumView v,
     const int ns = min(nsuper, (nblk + NBH_SUM_GROUP - 1) / NBH_SUM_GROUP);
     if (tid == 0) ncand = 0;
     __syncthreads();
-    for (int k = tid; k < ns; k += NBH_SPAN_THREADS) {
+    for (int k = tid; k < ns; k += NBH_SUM_THREADS) {
         const int c = span2_n[k];
         const int base = atomicAdd(&ncand, c);
         for (int j = 0; j < c; ++j) cand[base + j] = span2[(size_t) k * NBH_SPAN_SLOTS + j];
     }
     __syncthreads();
-    nbh_sum_handed<NBH_SPAN_THREADS>(v, cand, ncand, v.nn, nullptr, nullptr, list, cnt, off,
-                                     fill, &nspan, s_ch, scal);
+    nbh_sum_handed<NBH_SUM_THREADS, NBH_SUMT_KEEP>(v, cand, ncand, v.nn, nullptr, nullptr, list, lv, &nspan,
+                                     rec, terms, slot, scal);
 }
 
 /* The group walk's table from the finished summaries: one thread per node
@@ -1985,7 +2020,9 @@ void nbh_build(nbhip_state* st, int graph_safe)
     v.ctx = st->ctx;
     v.rc_scale = st->open_scale;
     v.nn = st->node_cap;
-    /* span: each block's spanning cells (NBH_SPAN_SLOTS each); span_sorted:
+    /* blist: over-long lists of k_sum_blocks, then each cell's place in the
+     * list of the pass that summarises it (other cells' entries are stale and
+     * rejected); span: each block's spanning cells (NBH_SPAN_SLOTS each); span_sorted:
      * each super-block's, then the per-block and per-super-block counts,
      * then the top launch's candidates and level-sorted list */
     const int nblk = nbh_blocks(n, NBH_SUM_BODIES);
@@ -1997,10 +2034,12 @@ void nbh_build(nbhip_state* st, int graph_safe)
     int* top_list = top_cand + (size_t) nsup * NBH_SPAN_SLOTS;
     hipLaunchKernelGGL(k_sum_blocks, dim3(nblk), dim3(NBH_SUMB_THREADS), 0, s, v, st->cincl,
                        st->blist, st->span, span_n, st->scal);
-    hipLaunchKernelGGL(k_sum_super, dim3(nsup), dim3(NBH_SUM_THREADS), 0, s, v, st->cincl,
-                       st->span, span_n, span2, span2_n, st->scal);
-    hipLaunchKernelGGL(k_sum_top, dim3(1), dim3(NBH_SPAN_THREADS), 0, s, v, span2, span2_n, nsup,
-                       top_cand, top_list, st->scal);
+    if (nblk > 1)
+        hipLaunchKernelGGL(k_sum_super, dim3(nsup), dim3(NBH_SUM_THREADS), 0, s, v, st->cincl,
+                           st->span, span_n, span2, span2_n, st->blist, st->scal);
+    if (nsup > 1)
+        hipLaunchKernelGGL(k_sum_top, dim3(1), dim3(NBH_SUM_THREADS), 0, s, v, span2, span2_n,
+                           nsup, top_cand, top_list, st->blist, st->scal);
     if (st->nodeg) {
         const GroupTab g{ st->nodeg, st->nkid, st->kbase, st->nsim };
         hipLaunchKernelGGL(k_group_table, dim3(nbh_blocks(st->node_cap, 256 * 4)), dim3(256), 0,
