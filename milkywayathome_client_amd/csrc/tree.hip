@@ -23,6 +23,7 @@
  * simulation's pre-order table is one contiguous segment.
  */
 #include <cstring>
+#include <utility>
 
 #include "nbhip_device.h"
 
@@ -170,43 +171,151 @@ __global__ __launch_bounds__(256) void k_rsize(int nsim, SimTab* __restrict__ si
 /* Sort word: simulation id above the top `top` Morton levels.  Massless
  * bodies are not inserted (nbMakeTree, nbody/src/nbody_tree.c:438-442):
  * their key sorts after every massive key. */
-__global__ __launch_bounds__(256) void k_keys(int n, const double* __restrict__ px,
-                                              const double* __restrict__ py,
-                                              const double* __restrict__ pz,
-                                              const double* __restrict__ m,
-                                              const int* __restrict__ simid,
-                                              const SimTab* __restrict__ sims, int sim_shift,
-                                              int top, unsigned long long* __restrict__ key,
+struct KeyView {
+    const double *px, *py, *pz, *m;
+    const int* simid;
+    const SimTab* sims;
+    int sim_shift, top;
+};
+__device__ __forceinline__ unsigned long long nbh_key(const KeyView& v, int i)
+{
+    unsigned long long k = ~0ull;
+    if (v.m[i] != 0.0) {
+        const int sim = v.simid[i];
+        const double ks = v.sims[sim].key_scale;
+        const int sh = 63 - v.top;
+        unsigned long long ux = nbh_fixed(v.px[i], ks);
+        unsigned long long uy = nbh_fixed(v.py[i], ks);
+        unsigned long long uz = nbh_fixed(v.pz[i], ks);
+        k = nbh_morton21(ux >> sh, uy >> sh, uz >> sh);
+        if (v.sim_shift < 64) k |= (unsigned long long) sim << v.sim_shift;
+    }
+    return k;
+}
+
+__global__ __launch_bounds__(256) void k_keys(int n, KeyView v,
+                                              unsigned long long* __restrict__ key,
                                               unsigned* __restrict__ perm)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    unsigned long long k = ~0ull;
-    if (m[i] != 0.0) {
-        const int sim = simid[i];
-        const double ks = sims[sim].key_scale;
-        const int sh = 63 - top;
-        unsigned long long ux = nbh_fixed(px[i], ks);
-        unsigned long long uy = nbh_fixed(py[i], ks);
-        unsigned long long uz = nbh_fixed(pz[i], ks);
-        k = nbh_morton21(ux >> sh, uy >> sh, uz >> sh);
-        if (sim_shift < 64) k |= (unsigned long long) sim << sim_shift;
-    }
-    key[i] = k;
+    key[i] = nbh_key(v, i);
     perm[i] = (unsigned) i;
 }
 
-/* Massive keys are < 2^63, massless keys all-ones: after the sort the
- * massive bodies are the prefix [0, M). */
-__global__ __launch_bounds__(256) void k_count_massive(int n,
-                                                       const unsigned long long* __restrict__ key,
-                                                       DevScalars* __restrict__ scal)
+/* ---------------------------------------------------------------------- */
+/* merge sort: tiles sorted by one workgroup each, then runs merged some at */
+/* a time, every element finding its own place                             */
+/* ---------------------------------------------------------------------- */
+/* States of up to NBH_MERGE_BODIES bodies.  24 launches of the radix sort,
+ * each a few microseconds however few the bodies, are what it costs there;
+ * the merges read every other run of their group a few lines at a time, which
+ * grows faster than the bodies.  Keys, sort, ties and gather, radix sort and
+ * merges: 108 and 14 us (10^3 bodies), 120 and 37 (2x10^4), 127 and 53 (10^5),
+ * 134 and 72 (2.6x10^5), 151 and 134 (5.2x10^5), 189 and 381 (10^6, fan 16).
+ * NBH_MERGE_FAN runs at once: 8 searches advance together; 6 cost a pass more
+ * at 4x10^4 (49 us to 38) and 2.6x10^5 (93 to 72), 12 and 16 search more for
+ * nothing at 10^5 (57 to 53), 32 at 2x10^4 (41 to 37). */
+#define NBH_MERGE_BODIES (1 << 19)
+#define NBH_MERGE_FAN 8
+/* Keys of NBH_MTILE bodies, sorted with their indices: a bitonic network of
+ * one element a thread, over shuffles up to 64 apart, through LDS beyond.
+ * (key, place in the tile) are distinct pairs, so the order is the stable
+ * one; places past n sort last (key all-ones, highest places). */
+#define NBH_MTILE 1024
+__global__ __launch_bounds__(NBH_MTILE) void k_sort_tiles(int n, KeyView v,
+                                                          unsigned long long* __restrict__ key,
+                                                          unsigned* __restrict__ perm)
+{
+    __shared__ unsigned long long s_key[NBH_MTILE];
+    __shared__ int s_at[NBH_MTILE];
+    const int t = threadIdx.x;
+    const int base = blockIdx.x * NBH_MTILE;
+    unsigned long long k = base + t < n ? nbh_key(v, base + t) : ~0ull;
+    int at = t;
+    #pragma unroll
+    for (int size = 2; size <= NBH_MTILE; size <<= 1) {
+        #pragma unroll
+        for (int d = size >> 1; d > 0; d >>= 1) {
+            unsigned long long ko;
+            int ao;
+            if (d >= 64) {
+                __syncthreads();                       /* the last exchange has been read */
+                s_key[t] = k;
+                s_at[t] = at;
+                __syncthreads();
+                ko = s_key[t ^ d];
+                ao = s_at[t ^ d];
+            } else {
+                ko = __shfl_xor(k, d, 64);
+                ao = __shfl_xor(at, d, 64);
+            }
+            const bool less = ko < k || (ko == k && ao < at);
+            const bool want_less = ((t & d) == 0) == ((t & size) == 0);
+            if (less == want_less) {
+                k = ko;
+                at = ao;
+            }
+        }
+    }
+    if (base + t < n) {
+        key[base + t] = k;
+        perm[base + t] = (unsigned) (base + at);
+    }
+}
+
+/* Runs of `len` sorted keys merged `fan` at a time: an element's place is its
+ * own in its run plus, for every other run of the group, the keys that come
+ * before it there -- equal ones count in earlier runs only, which keeps the
+ * order stable.  8 binary searches advance together (their loads overlap);
+ * the 64 elements of a wave follow each other in their run, so they probe a
+ * few cache lines of another. */
+__global__ __launch_bounds__(256) void k_sort_merge(int n, int len, int fan,
+                                                    const unsigned long long* __restrict__ kin,
+                                                    const unsigned* __restrict__ vin,
+                                                    unsigned long long* __restrict__ kout,
+                                                    unsigned* __restrict__ vout)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const bool massive = key[i] != ~0ull;
-    if (i == 0 && !massive) scal->nmassive = 0;
-    if (massive && (i + 1 == n || key[i + 1] == ~0ull)) scal->nmassive = i + 1;
+    const unsigned long long k = kin[i];
+    const unsigned val = vin[i];
+    const int run = i / len;
+    const int first = run / fan * fan;
+    const int last = min(first + fan, (n + len - 1) / len);
+    int half = 1;
+    while (2 * half <= len) half *= 2;
+    int at = first * len + (i - run * len);
+    for (int r0 = first; r0 < last; r0 += 8) {
+        int lo[8], m[8];
+        const unsigned long long* q[8];
+        bool tie[8];
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int r = r0 + j;
+            m[j] = r < last && r != run ? min(len, n - r * len) : 0;
+            q[j] = kin + (m[j] > 0 ? (size_t) r * len : 0);
+            tie[j] = r < run;
+            lo[j] = 0;
+        }
+        for (int step = half; step > 0; step >>= 1) {
+            unsigned long long x[8];
+            #pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int p = lo[j] + step;
+                x[j] = q[j][p <= m[j] ? p - 1 : 0];
+            }
+            #pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int p = lo[j] + step;
+                if (p <= m[j] && (x[j] < k || (tie[j] && x[j] == k))) lo[j] = p;
+            }
+        }
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) at += lo[j];
+    }
+    kout[at] = k;
+    vout[at] = val;
 }
 
 /* ---------------------------------------------------------------------- */
@@ -418,86 +527,64 @@ __device__ __forceinline__ bool nbh_words_gt(const unsigned long long* a,
     return a[2] > b[2];
 }
 
-__global__ __launch_bounds__(256) void k_tiefix_rank(const unsigned long long* __restrict__ key,
-                                                     const unsigned* __restrict__ perm,
-                                                     unsigned* __restrict__ perm_out,
-                                                     const double* __restrict__ px,
-                                                     const double* __restrict__ py,
-                                                     const double* __restrict__ pz,
-                                                     const int* __restrict__ simid,
-                                                     const SimTab* __restrict__ sims, int top,
-                                                     const DevScalars* __restrict__ scal)
+/* ---------------------------------------------------------------------- */
+/* sorted order: ties by the remaining levels, records of the sorted bodies */
+/* ---------------------------------------------------------------------- */
+/* Massive keys are < 2^63, massless keys all-ones: the massive bodies are the
+ * prefix [0, M) of the sorted ones.  A massive body whose key another one
+ * shares finds its place in the run of equal keys by the deeper levels; every
+ * body then writes its records (and perm) at its place.  One launch where
+ * count, ranking, copy-back and gather were four. */
+__global__ __launch_bounds__(256) void k_place(int n, const unsigned long long* __restrict__ key,
+                                               const unsigned* __restrict__ order, KeyView v,
+                                               const double4* __restrict__ pos4,
+                                               unsigned* __restrict__ perm,
+                                               double4* __restrict__ spos,
+                                               int* __restrict__ simid_s,
+                                               unsigned long long* __restrict__ su,
+                                               DevScalars* __restrict__ scal)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    const int M = scal->nmassive;
-    if (i >= M) return;
+    if (i >= n) return;
     const unsigned long long k = key[i];
-    const bool tie = (i > 0 && key[i - 1] == k) || (i + 1 < M && key[i + 1] == k);
-    if (!tie) return;
-    int a = i;
-    while (a > 0 && key[a - 1] == k) --a;
-    int e = i + 1;
-    while (e < M && key[e] == k) ++e;
-    const double ks = sims[simid[perm[i]]].key_scale;
-    unsigned long long wi[3];
-    nbh_deep_words(px, py, pz, ks, perm[i], top, wi);
-    /* rank in the run: members with smaller deeper words, and members with
-     * equal words that come earlier (the stable order of the sort) */
-    int rank = 0;
-    for (int j = a; j < e; ++j) {
-        if (j == i) continue;
-        unsigned long long wj[3];
-        nbh_deep_words(px, py, pz, ks, perm[j], top, wj);
-        if (nbh_words_gt(wi, wj) || (j < i && !nbh_words_gt(wj, wi))) ++rank;
-    }
-    perm_out[a + rank] = perm[i];
-}
-
-__global__ __launch_bounds__(256) void k_tiefix_copy(const unsigned long long* __restrict__ key,
-                                                     unsigned* __restrict__ perm,
-                                                     const unsigned* __restrict__ perm_out,
-                                                     const DevScalars* __restrict__ scal)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int M = scal->nmassive;
-    if (i >= M) return;
-    const unsigned long long k = key[i];
-    if ((i > 0 && key[i - 1] == k) || (i + 1 < M && key[i + 1] == k)) perm[i] = perm_out[i];
-}
-
-/* ---------------------------------------------------------------------- */
-/* sorted gather, adjacent prefixes, cells-per-first-body                  */
-/* ---------------------------------------------------------------------- */
-__global__ __launch_bounds__(256) void k_gather(int n, const unsigned* __restrict__ perm,
-                                                const double4* __restrict__ pos4,
-                                                const unsigned long long* __restrict__ key,
-                                                int sim_shift,
-                                                const int* __restrict__ simid,
-                                                const SimTab* __restrict__ sims,
-                                                double4* __restrict__ spos,
-                                                int* __restrict__ simid_s,
-                                                unsigned long long* __restrict__ su,
-                                                const DevScalars* __restrict__ scal)
-{
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= n) return;
-    const unsigned j = perm[s];
+    const unsigned j = order[i];
+    const unsigned long long after = i + 1 < n ? key[i + 1] : ~0ull;
+    const bool massive = k != ~0ull;
+    if (massive && after == ~0ull) scal->nmassive = i + 1;
     /* one 32-byte record per body; the simulation of a massive body is the
-     * top of its sorted key (massless bodies carry an all-ones key) */
+     * top of its key */
     const double4 p = pos4[j];
-    const double x = p.x, y = p.y, z = p.z;
-    const bool massive = s < scal->nmassive;
-    const int sim = (sim_shift >= 64) ? 0 : (massive ? (int) (key[s] >> sim_shift) : simid[j]);
+    const int sim = (v.sim_shift >= 64) ? 0 : (massive ? (int) (k >> v.sim_shift) : v.simid[j]);
+    int s = i;
+    if (massive) {
+        const double ks = v.sims[sim].key_scale;
+        if (after == k || (i > 0 && key[i - 1] == k)) {
+            int a = i;
+            while (a > 0 && key[a - 1] == k) --a;
+            unsigned long long wi[3];
+            nbh_deep_words(v.px, v.py, v.pz, ks, j, v.top, wi);
+            /* rank in the run: members with smaller deeper words, and members
+             * with equal words that come earlier (the stable order of the sort) */
+            s = a;
+            for (int e = a; e < n && key[e] == k; ++e) {
+                if (e == i) continue;
+                unsigned long long we[3];
+                nbh_deep_words(v.px, v.py, v.pz, ks, order[e], v.top, we);
+                if (nbh_words_gt(wi, we) || (e < i && !nbh_words_gt(we, wi))) ++s;
+            }
+        }
+        su[3 * (size_t) s + 0] = nbh_fixed(p.x, ks);
+        su[3 * (size_t) s + 1] = nbh_fixed(p.y, ks);
+        su[3 * (size_t) s + 2] = nbh_fixed(p.z, ks);
+    }
+    perm[s] = j;
     spos[s] = p;
     simid_s[s] = sim;
-    if (massive) {
-        const double ks = sims[sim].key_scale;
-        su[3 * (size_t) s + 0] = nbh_fixed(x, ks);
-        su[3 * (size_t) s + 1] = nbh_fixed(y, ks);
-        su[3 * (size_t) s + 2] = nbh_fixed(z, ks);
-    }
 }
 
+/* ---------------------------------------------------------------------- */
+/* adjacent prefixes, cells-per-first-body                                 */
+/* ---------------------------------------------------------------------- */
 /* Common prefix, in bits, of the full keys (simulation id in the top sb
  * bits, then the 189-bit Morton key) of sorted massive bodies i and j; -1
  * outside [0, M); equal keys ordered by index (Karras 2012, section 4). */
@@ -1944,34 +2031,53 @@ void nbh_build(nbhip_state* st, int graph_safe)
     const int g256 = nbh_blocks(n, 256);
     hipStream_t s = st->stream;
 
-    hipLaunchKernelGGL(k_keys, dim3(g256), dim3(256), 0, s, n, st->px, st->py, st->pz, st->m,
-                       st->simid, st->sims, st->sim_shift, st->top_levels, st->key, st->perm);
-    unsigned long long* kin = st->key;
-    unsigned long long* kout = st->key_alt;
-    unsigned* vin = st->perm;
-    unsigned* vout = st->perm_alt;
-    const int nb = st->sort_blocks;
-    for (int pass = 0; pass < 8; ++pass) {
-        const int shift = 8 * pass;
-        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(256), 0, s, n, shift, kin, st->hist, nb);
-        hipLaunchKernelGGL(k_radix_scan, dim3(256), dim3(256), 0, s, st->hist, st->dtot, nb);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(256), 0, s, n, shift, kin, vin, kout,
-                           vout, st->hist, st->dtot, nb);
-        unsigned long long* tk = kin; kin = kout; kout = tk;
-        unsigned* tv = vin; vin = vout; vout = tv;
+    const KeyView kv{ st->px, st->py, st->pz, st->m, st->simid, st->sims, st->sim_shift,
+                      st->top_levels };
+    /* the sorted order ends in key_alt / perm_alt, and k_place writes perm */
+    unsigned long long *kin = st->key_alt, *kout = st->key;
+    unsigned *vin = st->perm_alt, *vout = st->perm;
+    auto turn = [&]() {
+        std::swap(kin, kout);
+        std::swap(vin, vout);
+    };
+    if (n <= NBH_MERGE_BODIES) {
+        /* the fewest merges of at most NBH_MERGE_FAN runs, of equal fan */
+        const int tiles = nbh_blocks(n, NBH_MTILE);
+        int passes = 0, fan = 1;
+        for (long long cover = 1; cover < tiles; ++passes) cover *= NBH_MERGE_FAN;
+        if (passes) {
+            long long cover;
+            do {
+                ++fan;
+                cover = 1;
+                for (int k = 0; k < passes; ++k) cover *= fan;
+            } while (cover < tiles);
+        }
+        if (passes & 1) turn();
+        hipLaunchKernelGGL(k_sort_tiles, dim3(tiles), dim3(NBH_MTILE), 0, s, n, kv, kin, vin);
+        int len = NBH_MTILE;
+        for (int k = 0; k < passes; ++k, len *= fan) {
+            hipLaunchKernelGGL(k_sort_merge, dim3(g256), dim3(256), 0, s, n, len, fan, kin, vin,
+                               kout, vout);
+            turn();
+        }
+    } else {
+        const int nb = st->sort_blocks;
+        hipLaunchKernelGGL(k_keys, dim3(g256), dim3(256), 0, s, n, kv, kin, vin);
+        for (int pass = 0; pass < 8; ++pass) {
+            const int shift = 8 * pass;
+            hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(256), 0, s, n, shift, kin, st->hist,
+                               nb);
+            hipLaunchKernelGGL(k_radix_scan, dim3(256), dim3(256), 0, s, st->hist, st->dtot, nb);
+            hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(256), 0, s, n, shift, kin, vin,
+                               kout, vout, st->hist, st->dtot, nb);
+            turn();
+        }
     }
-    /* 8 passes: sorted data is back in st->key / st->perm */
-    hipLaunchKernelGGL(k_count_massive, dim3(g256), dim3(256), 0, s, n, st->key, st->scal);
-    /* perm_alt is free after the eighth pass */
-    hipLaunchKernelGGL(k_tiefix_rank, dim3(g256), dim3(256), 0, s, st->key, st->perm, st->perm_alt,
-                       st->px, st->py, st->pz, st->simid, st->sims, st->top_levels, st->scal);
-    hipLaunchKernelGGL(k_tiefix_copy, dim3(g256), dim3(256), 0, s, st->key, st->perm,
-                       st->perm_alt, st->scal);
     nbh_mark(st, 2);
 
-    hipLaunchKernelGGL(k_gather, dim3(g256), dim3(256), 0, s, n, st->perm, st->pos4, st->key,
-                       st->sim_shift, st->simid, st->sims, st->spos, st->simid_s, st->su,
-                       st->scal);
+    hipLaunchKernelGGL(k_place, dim3(g256), dim3(256), 0, s, n, st->key_alt, st->perm_alt, kv,
+                       st->pos4, st->perm, st->spos, st->simid_s, st->su, st->scal);
     hipLaunchKernelGGL(k_delta_count, dim3(g256), dim3(256), 0, s, n, st->su, st->simid_s,
                        st->dadj, st->cincl, st->sims, st->scal);
     const int nscan = nbh_blocks(n, NBH_SCAN_TILE);

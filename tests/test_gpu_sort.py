@@ -1,0 +1,51 @@
+"""The order of the sorted bodies against the oracle's tree (tolerance zero):
+body counts around a tile of 1024, the changes of the number of merges and of
+the sort; keys that tie in runs across tiles; massless bodies in between."""
+import numpy as np
+import pytest
+
+from helpers import plummer_bodies
+from milkywayathome_client_amd import nbody as nb
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(bodies, acc=False):
+    ctx = nb.NBodyCtx.create(timestep=1e-3, timeEvolve=1.0, eps2=1e-4, theta=1.0,
+                             criterion="bh86", useQuad=True, allowIncest=True)
+    o = orc.Oracle(orc.make_ctx(eps2=1e-4, theta=1.0, timestep=1e-3, allow_incest=True), *bodies)
+    o.gravity()
+    st = nb.NBodyState(ctx, None, *bodies)
+    gt, ct = st.tree(), o.tree()
+    a = st.accelerations() if acc else None
+    st.close()
+    assert gt["kind"].shape == ct["kind"].shape
+    leaf = ct["kind"] == 1
+    np.testing.assert_array_equal(gt["ref"][leaf], ct["ref"][leaf])
+    for k in ("kind", "skip", "level", "pos", "mass"):
+        np.testing.assert_array_equal(gt[k], ct[k], err_msg=k)
+    if acc:
+        np.testing.assert_array_equal(a, o.acc)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2047, 8191, 8192, 8193, 65535,
+                               65536, 65537, 524287, 524288, 524289])
+def test_body_counts(n):
+    _check(plummer_bodies(n, seed=n))
+
+
+@pytest.mark.parametrize("n,spread,run", [(700, 40.0, 300), (5000, 40.0, 2500), (5000, 0.0, 0)])
+@pytest.mark.parametrize("massless", [0, 3])
+def test_ties_and_massless_bodies(n, spread, run, massless):
+    """`run` bodies, from all over the input, share the first 22 levels."""
+    pos, vel, m = plummer_bodies(n, seed=3)
+    rng = np.random.default_rng(n)
+    pick = rng.choice(n, run, replace=False)
+    side = 4.0 * 2.0 ** -23
+    pos[pick] = np.array([3, 5, 7]) * side + rng.uniform(0.0, side, size=(run, 3))
+    pos[0] = spread                                   # a wide root
+    if massless:
+        m = m.copy()
+        m[1::massless] = 0.0
+    _check((pos, vel, m), acc=True)
