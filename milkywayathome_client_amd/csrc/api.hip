@@ -210,7 +210,8 @@ static unsigned nbh_create(const nbhip_ctx* ctx, int device, int nsim, const int
     A(hist, 256 * (size_t) st->sort_blocks);
     A(dtot, 256);
     A(pos4, n); A(spos, n); A(simid_s, n); A(su, 3 * n); A(dadj, nbh_dadj_cap(n)); A(cincl, n);
-    A(scan_part, std::max<size_t>(4096, (nc + NBH_SCAN_TILE - 1) / NBH_SCAN_TILE));
+    /* cells per 256 bodies, then children per tile of nodes */
+    A(scan_part, std::max<size_t>(n / 256 + 4, (nc + NBH_SCAN_TILE - 1) / NBH_SCAN_TILE));
     A(node, nc); A(nquad, 6 * nc); A(nmid, 3 * nc); A(nlevel, nc); A(nparent, nc);
     A(nsim_node, nc); A(level_list, nc); A(nnext, nc);
     if (ctx->precision == NBHIP_PRECISION_MIXED || ctx->precision == NBHIP_PRECISION_MIXED_COHERENT)

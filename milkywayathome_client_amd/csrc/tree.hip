@@ -22,6 +22,7 @@
  * tree is a forest joined by prefix -1 nodes (which own no cell) and each
  * simulation's pre-order table is one contiguous segment.
  */
+#include <algorithm>
 #include <cstring>
 #include <utility>
 
@@ -34,10 +35,12 @@
 /* ---------------------------------------------------------------------- */
 /* advancePosVel (nbody/src/nbody_plain.c:268-284) fused with expandBox's
  * max-|x| scan (nbody/src/nbody_tree.c:156-176), per simulation.  Each
- * block owns a contiguous chunk of NBH_BBOX_CHUNK bodies (coalesced, 256
- * apart per thread); a thread flushes its running maximum only when its
- * simulation changes, and waves then the block combine theirs, so a launch
- * issues about one atomic per block and simulation instead of one per wave.
+ * block owns a contiguous chunk of bodies (coalesced, 256 apart per
+ * thread); a thread flushes its running maximum only when its simulation
+ * changes, and waves then the block combine theirs, so a launch issues about
+ * one atomic per block and simulation instead of one per wave.  A chunk is
+ * NBH_BBOX_CHUNK bodies, fewer where that leaves under 256 workgroups: five
+ * chunks of 2x10^4 bodies took 17.5 us, 79 take 5.7.
  * A NaN coordinate counts as infinite so the root-size step reports it. */
 #define NBH_BBOX_CHUNK (256 * 16)
 
@@ -46,7 +49,8 @@ __device__ __forceinline__ void nbh_max_bits(SimTab* sims, int sim, double v)
     atomicMax(&sims[sim].xyzmax_bits, (unsigned long long) __double_as_longlong(v));
 }
 
-__global__ __launch_bounds__(256) void k_drift_bbox(int n, int drift, double dt, double dtHalf,
+__global__ __launch_bounds__(256) void k_drift_bbox(int n, int chunk, int drift, double dt,
+                                                    double dtHalf,
                                                     double* __restrict__ px, double* __restrict__ py,
                                                     double* __restrict__ pz, double* __restrict__ vx,
                                                     double* __restrict__ vy, double* __restrict__ vz,
@@ -62,8 +66,8 @@ __global__ __launch_bounds__(256) void k_drift_bbox(int n, int drift, double dt,
     __shared__ int s_sim[4];
     __shared__ double s_mx[4];
     if (scal->halt) return;               /* a fatal status stopped the run */
-    const int lo = blockIdx.x * NBH_BBOX_CHUNK;
-    const int hi = min(n, lo + NBH_BBOX_CHUNK);
+    const int lo = blockIdx.x * chunk;
+    const int hi = min(n, lo + chunk);
     int cur = -1;
     double mx = 0.0;
     for (int i = lo + (int) threadIdx.x; i < hi; i += 256) {
@@ -610,12 +614,14 @@ __device__ __forceinline__ bool nbh_first_of_sim(const int* __restrict__ simid_s
 __global__ __launch_bounds__(256) void k_delta_count(int n, const unsigned long long* __restrict__ su,
                                                      const int* __restrict__ simid_s,
                                                      int* __restrict__ dadj,
-                                                     unsigned* __restrict__ ccount,
+                                                     unsigned* __restrict__ cincl,
+                                                     unsigned* __restrict__ part,
                                                      SimTab* __restrict__ sims,
                                                      const DevScalars* __restrict__ scal)
 {
     __shared__ int bsim, bmax, mixed;
     __shared__ int s_min16[16];
+    __shared__ unsigned s_sum[4];
     if (threadIdx.x == 0) {
         bsim = -1;
         bmax = -1;
@@ -627,6 +633,7 @@ __global__ __launch_bounds__(256) void k_delta_count(int n, const unsigned long 
     const int sb = scal->sim_bits;
     int depth = -1, sim = -1;
     int hv = INT_MAX;                  /* this prefix in the min-hierarchy (none: +inf) */
+    unsigned cells = 0;
     if (a < M) {
         const int d = nbh_kdelta(su, simid_s, n, M, sb, a, a + 1);
         dadj[a] = d;
@@ -638,7 +645,7 @@ __global__ __launch_bounds__(256) void k_delta_count(int n, const unsigned long 
             const int dp = nbh_kdelta(su, simid_s, n, M, sb, a - 1, a);
             c = max(0, nbh_levels(d, sb) - nbh_levels(dp, sb));
         }
-        ccount[a] = (unsigned) c;
+        cells = (unsigned) c;
         depth = max(nbh_levels(d, sb), 0);
         sim = simid_s[a];
         if (threadIdx.x == 0) bsim = sim;
@@ -650,7 +657,18 @@ __global__ __launch_bounds__(256) void k_delta_count(int n, const unsigned long 
         if (h.top >= 1 && (a >> 4) < h.size[1]) dadj[h.off[1] + (a >> 4)] = hv;
         s_min16[threadIdx.x >> 4] = hv;
     }
+    /* the workgroup's running totals of cells (k_cells adds the workgroups
+     * before) */
+    unsigned incl = cells;
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned u = __shfl_up(incl, o, 64);
+        if ((int) __lane_id() >= o) incl += u;
+    }
+    if (__lane_id() == 63) s_sum[threadIdx.x >> 6] = incl;
     __syncthreads();
+    for (int w = 0; w < (int) threadIdx.x >> 6; ++w) incl += s_sum[w];
+    if (a < M) cincl[a] = incl;
+    if (threadIdx.x == 255) part[blockIdx.x] = incl;
     if (threadIdx.x == 0 && h.top >= 2 && (int) blockIdx.x < h.size[2]) {
         int bm = INT_MAX;
         for (int k = 0; k < 16; ++k) bm = min(bm, s_min16[k]);
@@ -670,9 +688,6 @@ __global__ __launch_bounds__(256) void k_delta_count(int n, const unsigned long 
         atomicMax(&sims[bsim].maxdepth, bmax);
 }
 
-/* ---------------------------------------------------------------------- */
-/* inclusive scan of cells-per-first-body (length nmassive)               */
-/* ---------------------------------------------------------------------- */
 __device__ __forceinline__ unsigned nbh_block1024_excl(unsigned s, unsigned* wsum,
                                                        unsigned* total)
 {
@@ -697,66 +712,13 @@ __device__ __forceinline__ unsigned nbh_block1024_excl(unsigned s, unsigned* wsu
     return v - s + ((t >> 6) ? wsum[(t >> 6) - 1] : 0u);
 }
 
-__global__ __launch_bounds__(1024) void k_scan_tiles(unsigned* __restrict__ data,
-                                                     unsigned* __restrict__ part,
-                                                     const DevScalars* __restrict__ scal)
-{
-    __shared__ unsigned wsum[16];
-    const int M = scal->nmassive;
-    const int base = blockIdx.x * NBH_SCAN_TILE + threadIdx.x * 4;
-    if (blockIdx.x * NBH_SCAN_TILE >= M) return;
-    unsigned v[4];
-    #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = (base + k < M) ? data[base + k] : 0u;
-    unsigned s = v[0] + v[1] + v[2] + v[3];
-    unsigned tot;
-    unsigned ex = nbh_block1024_excl(s, wsum, &tot);
-    #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        ex += v[k];
-        if (base + k < M) data[base + k] = ex;
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = tot;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_part(unsigned* __restrict__ part,
-                                                    const DevScalars* __restrict__ scal)
-{
-    __shared__ unsigned wsum[16];
-    const int M = scal->nmassive;
-    const int nb = (M + NBH_SCAN_TILE - 1) / NBH_SCAN_TILE;
-    const int base = threadIdx.x * 4;
-    unsigned v[4];
-    #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = (base + k < nb) ? part[base + k] : 0u;
-    unsigned s = v[0] + v[1] + v[2] + v[3];
-    unsigned tot;
-    unsigned ex = nbh_block1024_excl(s, wsum, &tot);
-    #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        ex += v[k];
-        if (base + k < nb) part[base + k] = ex;
-    }
-}
-
-__global__ __launch_bounds__(1024) void k_scan_add(unsigned* __restrict__ data,
-                                                   const unsigned* __restrict__ part,
-                                                   const DevScalars* __restrict__ scal)
-{
-    const int M = scal->nmassive;
-    if (blockIdx.x == 0) return;
-    const int base = blockIdx.x * NBH_SCAN_TILE + threadIdx.x * 4;
-    const unsigned add = part[blockIdx.x - 1];
-    #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (base + k < M) data[base + k] += add;
-}
-
 /* Exclusive scan of the children per node over the node table (length
- * scal->nnode): each cell's child block in the group walk table.  Tiles of
- * NBH_SCAN_TILE entries, then the tile totals (one workgroup, 4096 at a time
- * with a running carry), then the tile offsets added back.  A node table
- * that overflowed its capacity has no child counts: nothing is scanned. */
+ * scal->nnode): each cell's child block (kbase).  Tiles of NBH_SCAN_TILE
+ * entries here; k_fill_kids adds the tiles before, from their totals or, past
+ * NBH_KID_TILES tiles, from k_nscan_part's scan of them (one workgroup, 4096
+ * at a time with a running carry).  A node table that overflowed its capacity
+ * has no child counts: nothing is scanned. */
+#define NBH_KID_TILES 2048
 __device__ __forceinline__ int nbh_nscan_len(const DevScalars* scal, int node_cap)
 {
     if (scal->status & NBHIP_CELL_OVERFLOW_ERROR) return 0;
@@ -811,54 +773,86 @@ __global__ __launch_bounds__(1024) void k_nscan_part(unsigned* __restrict__ part
     }
 }
 
-__global__ __launch_bounds__(1024) void k_nscan_add(unsigned* __restrict__ out,
-                                                    const unsigned* __restrict__ part,
-                                                    int node_cap,
-                                                    const DevScalars* __restrict__ scal)
-{
-    const int nn = nbh_nscan_len(scal, node_cap);
-    if (blockIdx.x == 0 || blockIdx.x * NBH_SCAN_TILE >= nn) return;
-    const int base = blockIdx.x * NBH_SCAN_TILE + threadIdx.x * 4;
-    const unsigned add = part[blockIdx.x];
-    #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (base + k < nn) out[base + k] += add;
-}
-
 /* ---------------------------------------------------------------------- */
 /* node counts, per-simulation segments                                    */
 /* ---------------------------------------------------------------------- */
 
-/* Each simulation's first body (which owns its root cell) and root; thread 0 also finalises the cell
- * and node counts (cells = the inclusive scan's last entry) and flags a node
- * table overflow. */
-__global__ __launch_bounds__(256) void k_sim_roots(const int* __restrict__ simid_s,
-                                                   const unsigned* __restrict__ cincl,
-                                                   int node_cap, SimTab* __restrict__ sims,
-                                                   unsigned* __restrict__ nkid,
-                                                   DevScalars* __restrict__ scal)
+/* Finishes the running totals of cells per first body (k_delta_count's
+ * workgroups of 256): a wave takes such a tile, a thread four bodies.  With
+ * the totals known: each simulation's first body (which owns its root cell)
+ * and root, the child masks of the node table cleared for the emission, the
+ * cell and node counts and the flag of a table overflow from the last massive
+ * body -- with one simulation also its end and depth (k_sim_ends otherwise).
+ * The last workgroup builds the min-hierarchy's levels from 3 up.  One launch
+ * of 5 us (2x10^4 bodies) instead of six of 2.3 to 4.4, 14 at 10^6. */
+__global__ __launch_bounds__(256) void k_cells(int n, const int* __restrict__ simid_s,
+                                               unsigned* __restrict__ cincl,
+                                               const unsigned* __restrict__ part, int node_cap,
+                                               int nsim, SimTab* __restrict__ sims,
+                                               unsigned* __restrict__ nkid,
+                                               int* __restrict__ dadj,
+                                               DevScalars* __restrict__ scal)
 {
-    const int a = blockIdx.x * 256 + threadIdx.x;
-    if (a == 0) {
-        const int M = scal->nmassive;
-        const int C = M > 0 ? (int) cincl[M - 1] : 0;
-        const int nn = M + C;
-        scal->ncell = C;
-        scal->nnode = nn;
-        if (nn > node_cap) scal->status |= NBHIP_CELL_OVERFLOW_ERROR;
+    __shared__ unsigned s_sum[4];
+    const int t = threadIdx.x;
+    const int M = scal->nmassive;
+    if (blockIdx.x + 1 == gridDim.x) {
+        const NbhDHier h = nbh_dhier(n, M);
+        for (int L = 3; L <= h.top; ++L) {
+            for (int i = t; i < h.size[L]; i += 256) {
+                int m = INT_MAX;
+                for (int k = 0; k < 16; ++k) {
+                    const int c = 16 * i + k;
+                    if (c < h.size[L - 1]) m = min(m, dadj[h.off[L - 1] + c]);
+                }
+                dadj[h.off[L] + i] = m;
+            }
+            __syncthreads();
+        }
+        return;
     }
-    if (a >= scal->nmassive) return;
-    {
-        /* child counters of body a's new cells and its leaf (pre-order
-         * a + cincl[a-1] .. a + cincl[a]), counted by the emission */
-        const int lo = a + (a > 0 ? (int) cincl[a - 1] : 0);
-        const int hi = a + (int) cincl[a];
+    if (blockIdx.x * 1024 >= M) return;
+    const int tile = 4 * blockIdx.x + (t >> 6);
+    unsigned before = 0;
+    for (int i = t; i < 4 * (int) blockIdx.x; i += 256) before += part[i];
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if ((t & 63) == 0) s_sum[t >> 6] = before;
+    __syncthreads();
+    before = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+    for (int i = 4 * blockIdx.x; i < tile; ++i) before += i * 256 < M ? part[i] : 0u;
+    const int base = tile * 256 + 4 * (t & 63);
+    if (base >= M) return;
+    unsigned v[4];
+    #pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = base + k < M ? before + cincl[base + k] : 0u;
+    /* the total before the thread's first body: the lane before has it */
+    unsigned prev = __shfl_up(v[3], 1, 64);
+    if ((t & 63) == 0) prev = before;
+    #pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int a = base + k;
+        if (a >= M) break;
+        cincl[a] = v[k];
+        /* child masks of body a's new cells and its leaf, set by the emission */
+        const int lo = a + (int) prev, hi = a + (int) v[k];
         for (int i = lo; i <= hi && i < node_cap; ++i) nkid[i] = 0u;
+        const int sim = simid_s[a];
+        if (nbh_first_of_sim(simid_s, a)) {
+            sims[sim].first = a;
+            sims[sim].root = lo;
+        }
+        if (a == M - 1) {
+            const int nn = M + (int) v[k];
+            scal->ncell = (int) v[k];
+            scal->nnode = nn;
+            if (nn > node_cap) scal->status |= NBHIP_CELL_OVERFLOW_ERROR;
+            if (nsim == 1) {
+                sims[0].end = nn;
+                scal->maxdepth = sims[0].maxdepth;
+            }
+        }
+        prev = v[k];
     }
-    if (!nbh_first_of_sim(simid_s, a)) return;
-    const int k = simid_s[a];
-    sims[k].first = a;
-    sims[k].root = a + (a > 0 ? (int) cincl[a - 1] : 0);
 }
 
 __global__ __launch_bounds__(256) void k_sim_ends(int nsim, SimTab* __restrict__ sims,
@@ -911,27 +905,6 @@ __device__ __forceinline__ double nbh_rcrit2(const nbhip_ctx& c, double mx, doub
 /* ---------------------------------------------------------------------- */
 /* Karras binary radix tree (a forest across simulations)                  */
 /* ---------------------------------------------------------------------- */
-/* Levels 3 and up of the adjacent prefixes' min-hierarchy (levels 1 and 2
- * come from k_delta_count), one workgroup, level by level. */
-__global__ __launch_bounds__(1024) void k_dhier_top(int n, int* __restrict__ dadj,
-                                                    const DevScalars* __restrict__ scal)
-{
-    __shared__ NbhDHier h;
-    if (threadIdx.x == 0) h = nbh_dhier(n, scal->nmassive);
-    __syncthreads();
-    for (int L = 3; L <= h.top; ++L) {
-        for (int i = threadIdx.x; i < h.size[L]; i += 1024) {
-            int m = INT_MAX;
-            for (int t = 0; t < 16; ++t) {
-                const int c = 16 * i + t;
-                if (c < h.size[L - 1]) m = min(m, dadj[h.off[L - 1] + c]);
-            }
-            dadj[h.off[L] + i] = m;
-        }
-        __syncthreads();
-    }
-}
-
 /* Entries base .. base+15 of hierarchy level L below v (bit t: entry
  * base + t), entries past the level's end excluded; base is a multiple of
  * 16, so the chunk is four aligned 16-byte loads. */
@@ -1343,26 +1316,61 @@ __device__ __forceinline__ NodeG nbh_group_record(const NodeW& w, int c,
 
 /* Child lists: kid[kbase[p] .. kbase[p] + popcount(nkid[p])) holds the
  * children of cell p in octant order (nrank: a child's octant; nkid[p]: the
- * mask of occupied octants, both from the emission). */
+ * mask of occupied octants, both from the emission).  kbase is base (within
+ * tiles of NBH_SCAN_TILE nodes) plus the tile's offset: the totals of the
+ * tiles before, summed here, or part itself (scanned: past NBH_KID_TILES). */
 __global__ __launch_bounds__(256) void k_fill_kids(const int* __restrict__ nparent,
                                                    const int* __restrict__ nrank,
                                                    const unsigned* __restrict__ nkid,
-                                                   const unsigned* __restrict__ kbase,
+                                                   const unsigned* __restrict__ base,
+                                                   const unsigned* __restrict__ part, int scanned,
+                                                   unsigned* __restrict__ kbase,
                                                    int* __restrict__ kid, int node_cap,
                                                    DevScalars* __restrict__ scal)
 {
+    __shared__ unsigned s_off[NBH_KID_TILES];
+    __shared__ unsigned s_sum[4];
     if (scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) return;
     const int nn = min(scal->nnode, node_cap);
+    if (blockIdx.x * 256 >= nn) return;
+    if (!scanned) {
+        constexpr int PER = NBH_KID_TILES / 256;
+        const int t = threadIdx.x;
+        const int nt = (nn + NBH_SCAN_TILE - 1) / NBH_SCAN_TILE;
+        unsigned v[PER], sum = 0;
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            v[k] = t * PER + k < nt ? part[t * PER + k] : 0u;
+            sum += v[k];
+        }
+        unsigned x = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned u = __shfl_up(x, o, 64);
+            if ((int) __lane_id() >= o) x += u;
+        }
+        if (__lane_id() == 63) s_sum[t >> 6] = x;
+        __syncthreads();
+        for (int w = 0; w < t >> 6; ++w) x += s_sum[w];
+        x -= sum;
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            s_off[t * PER + k] = x;
+            x += v[k];
+        }
+        __syncthreads();
+    }
+    auto off = [&](int q) { return scanned ? part[q / NBH_SCAN_TILE] : s_off[q / NBH_SCAN_TILE]; };
     for (int q = blockIdx.x * 256 + threadIdx.x; q < nn; q += gridDim.x * 256) {
+        kbase[q] = base[q] + off(q);
         const int par = nparent[q];
         if (par < 0) continue;
         const int r = nrank[q];
-        const unsigned mask = nkid[par];
+        const unsigned mask = par < q ? nkid[par] : 0u;
         if (par >= q || r < 0 || r > 7 || !((mask >> r) & 1u)) {
             atomicOr(&scal->status, NBHIP_ERROR);
             continue;
         }
-        kid[kbase[par] + __popc(mask & ((1u << r) - 1u))] = q;
+        kid[base[par] + off(par) + __popc(mask & ((1u << r) - 1u))] = q;
     }
 }
 
@@ -1944,10 +1952,10 @@ static inline int nbh_blocks(int n, int per) { return n > 0 ? (n + per - 1) / pe
 void nbh_bbox(nbhip_state* st, int drift)
 {
     const double dt = st->ctx.timestep;
-    hipLaunchKernelGGL(k_drift_bbox, dim3(nbh_blocks(st->n, NBH_BBOX_CHUNK)), dim3(256), 0,
-                       st->stream,
-                       st->n, drift, dt, 0.5 * dt, st->px, st->py, st->pz, st->vx, st->vy, st->vz,
-                       st->ax, st->ay, st->az, st->m, st->pos4, st->simid, st->sims, st->scal);
+    const int chunk = std::min(NBH_BBOX_CHUNK, std::max(256, nbh_blocks(st->n, 256 * 256) * 256));
+    hipLaunchKernelGGL(k_drift_bbox, dim3(nbh_blocks(st->n, chunk)), dim3(256), 0, st->stream,
+                       st->n, chunk, drift, dt, 0.5 * dt, st->px, st->py, st->pz, st->vx, st->vy,
+                       st->vz, st->ax, st->ay, st->az, st->m, st->pos4, st->simid, st->sims, st->scal);
     hipLaunchKernelGGL(k_rsize, dim3(1), dim3(256), 0, st->stream, st->nsim, st->sims, st->scal);
 }
 
@@ -2079,17 +2087,12 @@ void nbh_build(nbhip_state* st, int graph_safe)
     hipLaunchKernelGGL(k_place, dim3(g256), dim3(256), 0, s, n, st->key_alt, st->perm_alt, kv,
                        st->pos4, st->perm, st->spos, st->simid_s, st->su, st->scal);
     hipLaunchKernelGGL(k_delta_count, dim3(g256), dim3(256), 0, s, n, st->su, st->simid_s,
-                       st->dadj, st->cincl, st->sims, st->scal);
-    const int nscan = nbh_blocks(n, NBH_SCAN_TILE);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(nscan), dim3(1024), 0, s, st->cincl, st->scan_part,
-                       st->scal);
-    hipLaunchKernelGGL(k_scan_part, dim3(1), dim3(1024), 0, s, st->scan_part, st->scal);
-    hipLaunchKernelGGL(k_scan_add, dim3(nscan), dim3(1024), 0, s, st->cincl, st->scan_part,
-                       st->scal);
-    hipLaunchKernelGGL(k_sim_roots, dim3(g256), dim3(256), 0, s, st->simid_s, st->cincl,
-                       st->node_cap, st->sims, st->nkid, st->scal);
-    hipLaunchKernelGGL(k_sim_ends, dim3(1), dim3(256), 0, s, st->nsim, st->sims, st->scal);
-    hipLaunchKernelGGL(k_dhier_top, dim3(1), dim3(1024), 0, s, n, st->dadj, st->scal);
+                       st->dadj, st->cincl, st->scan_part, st->sims, st->scal);
+    hipLaunchKernelGGL(k_cells, dim3(nbh_blocks(n, 1024) + 1), dim3(256), 0, s, n, st->simid_s,
+                       st->cincl, st->scan_part, st->node_cap, st->nsim, st->sims, st->nkid,
+                       st->dadj, st->scal);
+    if (st->nsim > 1)
+        hipLaunchKernelGGL(k_sim_ends, dim3(1), dim3(256), 0, s, st->nsim, st->sims, st->scal);
     hipLaunchKernelGGL(k_emit_cells, dim3(g256), dim3(256), 0, s, n, st->dadj, st->cincl,
                        st->su, st->simid_s, st->nmid, st->nlevel, st->nparent, st->nsim_node,
                        st->sims, st->nkid, st->nrank, st->nnext, st->scal);
@@ -2099,15 +2102,16 @@ void nbh_build(nbhip_state* st, int graph_safe)
                        st->nkid, st->nrank, st->nnext, st->scal);
     /* each cell's child block (kbase) and child list (kid) */
     const int nt = nbh_blocks(st->node_cap, NBH_SCAN_TILE);
-    hipLaunchKernelGGL(k_nscan_tiles, dim3(nt), dim3(1024), 0, s, st->nkid, st->kbase,
+    unsigned* kid_base = reinterpret_cast<unsigned*>(st->blist);   /* free until the summaries */
+    const int scanned = nt > NBH_KID_TILES;
+    hipLaunchKernelGGL(k_nscan_tiles, dim3(nt), dim3(1024), 0, s, st->nkid, kid_base,
                        st->scan_part, st->node_cap, st->scal);
-    hipLaunchKernelGGL(k_nscan_part, dim3(1), dim3(1024), 0, s, st->scan_part, st->node_cap,
-                       st->scal);
-    hipLaunchKernelGGL(k_nscan_add, dim3(nt), dim3(1024), 0, s, st->kbase, st->scan_part,
-                       st->node_cap, st->scal);
+    if (scanned)
+        hipLaunchKernelGGL(k_nscan_part, dim3(1), dim3(1024), 0, s, st->scan_part, st->node_cap,
+                           st->scal);
     hipLaunchKernelGGL(k_fill_kids, dim3(nbh_blocks(st->node_cap, 256 * 8)), dim3(256), 0, s,
-                       st->nparent, st->nrank, st->nkid, st->kbase, st->kid, st->node_cap,
-                       st->scal);
+                       st->nparent, st->nrank, st->nkid, kid_base, st->scan_part, scanned,
+                       st->kbase, st->kid, st->node_cap, st->scal);
     nbh_mark(st, 3);
     /* level lists are built only for the adjoint's top-down pass (on its
      * request: nbh_level_lists) */

@@ -1,6 +1,8 @@
-"""The order of the sorted bodies against the oracle's tree (tolerance zero):
-body counts around a tile of 1024, the changes of the number of merges and of
-the sort; keys that tie in runs across tiles; massless bodies in between."""
+"""The order of the sorted bodies and the cells' places against the oracle's
+tree (tolerance zero): body counts around a tile of 1024, the changes of the
+number of merges and of the sort, and the most node tiles whose offsets are
+summed in place; keys that tie in runs across tiles; massless bodies in
+between."""
 import numpy as np
 import pytest
 
@@ -30,7 +32,7 @@ def _check(bodies, acc=False):
 
 
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2047, 8191, 8192, 8193, 65535,
-                               65536, 65537, 524287, 524288, 524289])
+                               65536, 65537, 524287, 524288, 524289, 1677516, 1677517])
 def test_body_counts(n):
     _check(plummer_bodies(n, seed=n))
 
