@@ -107,7 +107,7 @@ static void nbh_free_all(nbhip_state* st)
                      st->exact_part, st->nodeg, st->nkid, st->kbase, st->best_buf,
                      st->nrank, st->kid, st->blist, st->span, st->span_sorted, st->gcost,
                      st->gorder, st->bcost, st->gtask, st->nnext, st->bbox,
-                     st->wlist, st->wlen };
+                     st->wlist, st->wlen, st->wsum, st->wmet };
     for (void* p : ptrs)
         if (p) (void) hipFree(p);
     if (st->graph_exec) (void) hipGraphExecDestroy(st->graph_exec);
@@ -233,6 +233,12 @@ static unsigned nbh_create(const nbhip_ctx* ctx, int device, int nsim, const int
         const size_t ng = ((size_t) st->n + 63) / 64 + 1;
         A(wlist, ng * NBH_LIST_CAP);
         A(wlen, ng);
+    }
+    if ((ctx->precision == NBHIP_PRECISION_MIXED ||
+         ctx->precision == NBHIP_PRECISION_MIXED_COHERENT) &&
+        ctx->criterion != NBHIP_EXACT && st->n > 0 && st->n <= NBH_PIECE_BODIES) {
+        A(wsum, 6 * (size_t) NBH_PIECES * st->n);
+        A(wmet, (size_t) NBH_PIECES * st->n);
     }
     A(nkid, nc); A(kbase, nc); A(nrank, nc); A(kid, nc); A(blist, nc); A(span, nc);
     A(span_sorted, nc);

@@ -157,6 +157,15 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
 #define NBH_LIST_BODIES (1 << 17)
 #define NBH_LIST_WIDE 8192
 
+/* Mixed and coherent walks of at most NBH_PIECE_BODIES bodies are cut into
+ * NBH_PIECES parts (8 and 16 parts, one wave, us per mixed walk: 2x10^4
+ * bodies 312, 230, 836; 10^5 740, 689, 1196; 2x10^5 1230, 1136, 1573; 4x10^5
+ * 2184, 2198, 2289; at 10^6 8 parts 5433, one wave 5154).  The 16 waves of
+ * the same bodies in one workgroup instead: 2450 at 10^5 -- waves that walk
+ * the same nodes have to share a scalar cache.  Consecutive workgroups on
+ * consecutive XCDs instead of one stretch of bodies an XCD: 810. */
+#define NBH_PIECES 16
+#define NBH_PIECE_BODIES (1 << 18)
 #define NBH_SORT_TILE 2048   /* keys per radix-sort block: 256 threads x 8 */
 #define NBH_SCAN_TILE 4096   /* items per scan block: 1024 threads x 4 */
 
@@ -231,6 +240,8 @@ struct nbhip_state {
     int *span, *span_sorted;      /* summaries: cells spanning body blocks / super-blocks */
     int *wlist, *wlen;            /* FP64 list walk: each 64-body group's nodes in pre-order
                                      (NBH_LIST_CAP slots) and their count, -1: streaming walk */
+    double *wsum;                 /* mixed walk in parts: each part's sums and their errors */
+    unsigned *wmet;               /* and 0 where a body met its own record */
     double *exact_part;           /* Exact criterion: per-segment partial sums */
     int exact_seg;                /* Exact criterion: most segments of any simulation */
 

@@ -64,6 +64,22 @@ __device__ __forceinline__ void nbh_walk_counters(DevScalars* scal, unsigned nbb
     }
 }
 
+/* sum += v with the rounding error kept in err (Knuth's TwoSum): while the
+ * errors themselves add without rounding -- FP32 values over some 70 bits of
+ * exponent -- sum + err is the exact total, whatever the order. */
+__device__ __forceinline__ void nbh_exact_add(double& sum, double& err, double v)
+{
+    const double t = sum + v;
+    const double b = t - sum;
+    err += (sum - (t - b)) + (v - b);
+    sum = t;
+}
+/* The total, rounded once (an infinite sum has no error term). */
+__device__ __forceinline__ double nbh_exact_total(double sum, double err)
+{
+    return err == err ? sum + err : sum;
+}
+
 /* Kahan-compensated FP64 accumulation of FP32 partial sums. */
 __device__ __forceinline__ void nbh_kahan_add(double& sum, double& comp, double v)
 {

@@ -151,7 +151,8 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
 
 /* Mixed form: displacements and interactions in FP32; FP32 partial sums
  * per block of 2^batch_shift pre-order node indices (counted from the
- * body's own simulation root), added into FP64 with Kahan compensation.
+ * body's own simulation root), added in FP64 with the rounding errors kept
+ * (nbh_exact_add), so that the total does not depend on the order.
  * Positions, potential and kicks stay FP64.
  *
  * The walk is two nested loops: the inner one streams nodes until the wave
@@ -161,13 +162,22 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
  * property of its own interaction list, not of the wave -- and the FP64
  * state is not touched in the inner loop.
  *
+ * SPLIT: the walk of a wave is a chain of dependent loads, tests and votes,
+ * ~900 cycles a node, and states of up to NBH_PIECE_BODIES bodies have too
+ * few waves to cover it (10^5: 1.5 a SIMD).  Then NBH_PIECES waves share the
+ * bodies' walk: each takes an equal run of the simulation's node blocks and
+ * first goes from the root to its first block, some 30 nodes; k_walk_fold
+ * adds the parts.  Exact sums of the same FP32 partials: a body's result is
+ * the one that a single wave gives.  Waves that hold several simulations are
+ * not split.  Figures at NBH_PIECES.
+ *
  * COH selects the opening rule: false = each lane's own reference decision
  * (the FP64 walk's interaction lists); true = wave-coherent, the wave opens
  * a node when any lane's criterion says open and otherwise every lane of the
  * node's simulation interacts with it (each lane's list then refines its
  * reference list: every accepted node passes that lane's own test). */
 
-template <int BS, bool QUAD, bool COUNT, bool COH, bool MULTI, bool EPS0>
+template <int BS, bool SPLIT, bool QUAD, bool COUNT, bool COH, bool MULTI, bool EPS0>
 __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
                                                const NodeW* __restrict__ nodew,
                                                const double4* __restrict__ spos,
@@ -180,9 +190,15 @@ __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
                                                double* __restrict__ vx,
                                                double* __restrict__ vy,
                                                double* __restrict__ vz,
-                                               DevScalars* __restrict__ scal, WalkOut o)
+                                               DevScalars* __restrict__ scal,
+                                               double* __restrict__ wsum,
+                                               unsigned* __restrict__ wmet, WalkOut o)
 {
-    const int s = blockIdx.x * BS + threadIdx.x;
+    const int piece = SPLIT ? (int) blockIdx.y : 0;
+    /* an XCD's share of a split launch is one stretch of the sorted bodies */
+    const int bx = SPLIT ? (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3)
+                         : (int) blockIdx.x;
+    const int s = bx * BS + threadIdx.x;
     if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
     const int M = scal->nmassive;
     const bool valid = s < o.n;
@@ -211,6 +227,41 @@ __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
      * interaction.  The successor lies in [q + 1, qend], so every step
      * advances and every fetch stays inside the table (it holds one record
      * past the last node); the summaries already reject broken Next links. */
+    /* this wave's part of the walk: [q, stop) */
+    int stop = qend;
+    if (SPLIT) {
+        if (!one_root) {
+            if (piece > 0) stop = q;               /* several roots: the first wave walks alone */
+        } else if (q < qend) {
+            const int blocks = ((qend - 1 - root_u) >> bshift) + 1;
+            const int from = root_u + ((int) ((long long) blocks * piece / NBH_PIECES) << bshift);
+            if (piece + 1 < NBH_PIECES)
+                stop = root_u + ((int) ((long long) blocks * (piece + 1) / NBH_PIECES) << bshift);
+            if (from >= stop) stop = q;            /* fewer blocks than parts */
+            /* to `from`: over everything that ends before it, down into the
+             * cells that hold it; those accepted count in an earlier part */
+            while (q < from && q < stop) {
+                const NodeF nd = node[q];
+                const bool over = nd.next <= from;
+                const float dx = (float) (nd.x - p.x);
+                const float dy = (float) (nd.y - p.y);
+                const float dz = (float) (nd.z - p.z);
+                const float drSq = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                bool any_open;
+                if (COH) {
+                    const unsigned long long pass = __builtin_amdgcn_fcmpf(drSq, nd.rcrit2, 3);
+                    any_open = (valid_m & ~pass) != 0ull;
+                } else {
+                    const bool opn = lp == q && !over && !(drSq >= nd.rcrit2);
+                    any_open = __builtin_amdgcn_ballot_w64(opn) != 0ull;
+                    if (lp == q) lp = opn ? q + 1 : nd.next;
+                    if (MULTI && lp >= my_end) lp = INT_MAX;
+                }
+                q = min(max(!over && any_open ? q + 1 : nd.next, q + 1), qend);
+            }
+        }
+    }
+
     auto step = [&](const NodeF& nd, NodeF& nxt) {
         if (COUNT) ++steps;
         const float dx = (float) (nd.x - p.x);
@@ -271,7 +322,7 @@ __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
 
     NodeF nda = node[min(max(q, 0), qend)];
     NodeF ndb;
-    while (q < qend) {
+    while (q < stop) {
         /* nearest block boundary above q among the lanes' own blocks */
         int lim;
         if (one_root) {
@@ -299,20 +350,80 @@ __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
         const int rb = one_root ? root_u : root;
         const bool crossed = ((q - rb) >> bshift) != ((qstart - rb) >> bshift);
         if (crossed && (sx != 0.0f || sy != 0.0f || sz != 0.0f)) {
-            nbh_kahan_add(ax, cx, (double) sx);
-            nbh_kahan_add(ay, cy, (double) sy);
-            nbh_kahan_add(az, cz, (double) sz);
+            nbh_exact_add(ax, cx, (double) sx);
+            nbh_exact_add(ay, cy, (double) sy);
+            nbh_exact_add(az, cz, (double) sz);
             sx = sy = sz = 0.0f;
         }
     }
-    nbh_kahan_add(ax, cx, (double) sx);
-    nbh_kahan_add(ay, cy, (double) sy);
-    nbh_kahan_add(az, cz, (double) sz);
+    nbh_exact_add(ax, cx, (double) sx);
+    nbh_exact_add(ay, cy, (double) sy);
+    nbh_exact_add(az, cz, (double) sz);
+
+    if (SPLIT) {
+        if (!valid) return;
+        double* const a = wsum + 6 * (size_t) o.n * piece + s;
+        a[0] = ax;
+        a[(size_t) o.n] = ay;
+        a[2 * (size_t) o.n] = az;
+        a[3 * (size_t) o.n] = cx;
+        a[4 * (size_t) o.n] = cy;
+        a[5 * (size_t) o.n] = cz;
+        wmet[(size_t) o.n * piece + s] = metv;
+        return;
+    }
+    ax = nbh_exact_total(ax, cx);
+    ay = nbh_exact_total(ay, cy);
+    az = nbh_exact_total(az, cz);
 
     if (COUNT) nbh_walk_counters(scal, nbb, nbc, nop, steps);
     if (!valid) return;
     if (metv != 0u) atomicOr(&sims[L.sim].incest, 1u);
     nbh_walk_finish(o, p.x, p.y, p.z, ax, ay, az, perm[s], oax, oay, oaz, vx, vy, vz);
+}
+
+/* The parts of a split mixed walk added up, and the step finished: 816 bytes
+ * read per body, consecutive lanes consecutive addresses. */
+__global__ __launch_bounds__(256) void k_walk_fold(const double* __restrict__ wsum,
+                                                   const unsigned* __restrict__ wmet,
+                                                   const double4* __restrict__ spos,
+                                                   const unsigned* __restrict__ perm,
+                                                   const int* __restrict__ simid_s,
+                                                   SimTab* __restrict__ sims,
+                                                   double* __restrict__ oax,
+                                                   double* __restrict__ oay,
+                                                   double* __restrict__ oaz,
+                                                   double* __restrict__ vx,
+                                                   double* __restrict__ vy,
+                                                   double* __restrict__ vz,
+                                                   const DevScalars* __restrict__ scal, WalkOut o)
+{
+    const int s = blockIdx.x * 256 + threadIdx.x;
+    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    if (s >= o.n) return;
+    const size_t n = (size_t) o.n;
+    double part[NBH_PIECES][6];
+    unsigned metv = ~0u;
+    #pragma unroll
+    for (int k = 0; k < NBH_PIECES; ++k) {
+        #pragma unroll
+        for (int j = 0; j < 6; ++j) part[k][j] = wsum[(6 * k + j) * n + s];
+        metv = min(metv, wmet[k * n + s]);
+    }
+    const double4 p = spos[s];
+    double a[3] = { part[0][0], part[0][1], part[0][2] };
+    double c[3] = { part[0][3], part[0][4], part[0][5] };
+    #pragma unroll
+    for (int k = 1; k < NBH_PIECES; ++k) {
+        #pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            nbh_exact_add(a[j], c[j], part[k][j]);
+            c[j] += part[k][3 + j];
+        }
+    }
+    if (metv != 0u) atomicOr(&sims[simid_s[s]].incest, 1u);
+    nbh_walk_finish(o, p.x, p.y, p.z, nbh_exact_total(a[0], c[0]), nbh_exact_total(a[1], c[1]),
+                    nbh_exact_total(a[2], c[2]), perm[s], oax, oay, oaz, vx, vy, vz);
 }
 
 /* FP64 direct-sum checker on sampled bodies: one block per sample, the
@@ -394,26 +505,39 @@ void nbh_walk(nbhip_state* st, int kick, int count, double* oax, double* oay, do
     dim3 grid(nbh_blocks(st->n, bs)), block(bs);
     if (c.precision != NBHIP_PRECISION_FP64) {
         const bool coherent = c.precision == NBHIP_PRECISION_MIXED_COHERENT;
-#define NBH_W32E(B, Q, C, H, MU, E0)                                                         \
-    hipLaunchKernelGGL((k_walk32<B, Q, C, H, MU, E0>), grid, block, 0, s, st->nodef, st->node, \
+        const bool pieces = st->wsum && !count;
+        if (pieces) grid = dim3((grid.x + 7) / 8 * 8, NBH_PIECES);
+#define NBH_W32E(B, P, Q, C, H, MU, E0)                                                      \
+    hipLaunchKernelGGL((k_walk32<B, P, Q, C, H, MU, E0>), grid, block, 0, s, st->nodef, st->node, \
                        st->spos, st->perm, st->simid_s, st->sims, oax, oay, oaz, st->vx,       \
-                       st->vy, st->vz, st->scal, o)
-#define NBH_W32M(B, Q, C, H, MU)                                                             \
-    do { if (o.all_eps2_pos) NBH_W32E(B, Q, C, H, MU, false);                                 \
-         else NBH_W32E(B, Q, C, H, MU, true); } while (0)
-#define NBH_W32C(B, Q, C, H)                                                                 \
-    do { if (o.multi) NBH_W32M(B, Q, C, H, true); else NBH_W32M(B, Q, C, H, false); } while (0)
-#define NBH_W32(B, Q, C)                                                                     \
-    do { if (coherent) NBH_W32C(B, Q, C, true); else NBH_W32C(B, Q, C, false); } while (0)
+                       st->vy, st->vz, st->scal, st->wsum, st->wmet, o)
+#define NBH_W32M(B, P, Q, C, H, MU)                                                             \
+    do { if (o.all_eps2_pos) NBH_W32E(B, P, Q, C, H, MU, false);                                 \
+         else NBH_W32E(B, P, Q, C, H, MU, true); } while (0)
+#define NBH_W32C(B, P, Q, C, H)                                                                 \
+    do { if (o.multi) NBH_W32M(B, P, Q, C, H, true); else NBH_W32M(B, P, Q, C, H, false); } while (0)
+#define NBH_W32(B, P, Q, C)                                                                     \
+    do { if (coherent) NBH_W32C(B, P, Q, C, true); else NBH_W32C(B, P, Q, C, false); } while (0)
 #define NBH_W32B(B)                                                                          \
-    if (c.use_quad) { if (count) NBH_W32(B, true, true); else NBH_W32(B, true, false); }     \
-    else { if (count) NBH_W32(B, false, true); else NBH_W32(B, false, false); }
+    if (c.use_quad) {                                                                        \
+        if (pieces) NBH_W32(B, true, true, false);                                            \
+        else if (count) NBH_W32(B, false, true, true);                                        \
+        else NBH_W32(B, false, true, false);                                                  \
+    } else {                                                                                 \
+        if (pieces) NBH_W32(B, true, false, false);                                           \
+        else if (count) NBH_W32(B, false, false, true);                                       \
+        else NBH_W32(B, false, false, false);                                                 \
+    }
         if (bs == 64) { NBH_W32B(64) } else if (bs == 128) { NBH_W32B(128) } else { NBH_W32B(256) }
 #undef NBH_W32B
 #undef NBH_W32
 #undef NBH_W32C
 #undef NBH_W32M
 #undef NBH_W32E
+        if (pieces)
+            hipLaunchKernelGGL(k_walk_fold, dim3(nbh_blocks(st->n, 256)), dim3(256), 0, s, st->wsum,
+                               st->wmet, st->spos, st->perm, st->simid_s, st->sims, oax, oay, oaz,
+                               st->vx, st->vy, st->vz, st->scal, o);
         return;
     }
     /* small states: interaction lists, then the streaming walk for the groups
