@@ -249,8 +249,21 @@ static unsigned nbh_create(const nbhip_ctx* ctx, int device, int nsim, const int
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&st->stream, hipStreamNonBlocking);
     for (int k = 0; k < 6 && e == hipSuccess; ++k) e = hipEventCreate(&st->ev[k]);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&st->ev_counts, hipEventDisableTiming);
-    if (e == hipSuccess)
-        e = hipHostMalloc((void**) &st->h_counts_pinned, 64 * sizeof(int), hipHostMallocDefault);
+    if (e == hipSuccess) {
+        /* one page-locked block, its parts on 256-byte boundaries */
+        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        const size_t o_scal = up(64 * sizeof(int)), o_sims = o_scal + up(sizeof(DevScalars)),
+                     o_body = o_sims + up(nsim * sizeof(SimTab));
+        const bool small = n > 0 && n <= NBH_PINNED_BODIES;
+        e = hipHostMalloc((void**) &st->h_pinned, o_body + (small ? 9 * n * sizeof(double) : 0),
+                          hipHostMallocDefault);
+        if (e == hipSuccess) {
+            st->h_counts_pinned = reinterpret_cast<int*>(st->h_pinned);
+            st->h_scal = reinterpret_cast<DevScalars*>(st->h_pinned + o_scal);
+            st->h_sims = reinterpret_cast<SimTab*>(st->h_pinned + o_sims);
+            if (small) st->h_bodies = reinterpret_cast<double*>(st->h_pinned + o_body);
+        }
+    }
     if (e != hipSuccess) {
         nbh_set_error("allocation for %d bodies failed: %s", st->n, hipGetErrorString(e));
         nbh_free_all(st);
@@ -291,7 +304,7 @@ extern "C" void nbhip_release(nbhip_state* st)
     for (int k = 0; k < 6; ++k)
         if (st->ev[k]) (void) hipEventDestroy(st->ev[k]);
     if (st->ev_counts) (void) hipEventDestroy(st->ev_counts);
-    if (st->h_counts_pinned) (void) hipHostFree(st->h_counts_pinned);
+    if (st->h_pinned) (void) hipHostFree(st->h_pinned);
     if (st->stream) (void) hipStreamDestroy(st->stream);
     nbh_free_all(st);
     free(st);
@@ -303,15 +316,13 @@ static unsigned nbh_upload_range(nbhip_state* st, int off, int cnt, const double
     NBH_CHECK(hipSetDevice(st->device));
     const size_t n = (size_t) cnt;
     if (n == 0) return NBHIP_SUCCESS;
-    std::vector<double> tmp(n);
-    double* dst[6] = { st->px, st->py, st->pz, st->vx, st->vy, st->vz };
-    for (int k = 0; k < 6; ++k) {
-        const double* src = k < 3 ? pos : vel;
-        const int d = k % 3;
-        for (size_t i = 0; i < n; ++i) tmp[i] = src[3 * i + d];
-        NBH_CHECK(hipMemcpyAsync(dst[k] + off, tmp.data(), n * sizeof(double),
+    /* su is scratch of the tree build */
+    double* triples = reinterpret_cast<double*>(st->su);
+    for (int k = 0; k < 2; ++k) {
+        NBH_CHECK(hipMemcpyAsync(triples, k ? vel : pos, 3 * n * sizeof(double),
                                  hipMemcpyHostToDevice, st->stream));
-        NBH_CHECK(hipStreamSynchronize(st->stream));
+        if (k) nbh_unpack3(st->stream, cnt, triples, st->vx + off, st->vy + off, st->vz + off);
+        else nbh_unpack3(st->stream, cnt, triples, st->px + off, st->py + off, st->pz + off);
     }
     NBH_CHECK(hipMemcpyAsync(st->m + off, mass, n * sizeof(double), hipMemcpyHostToDevice,
                              st->stream));
@@ -327,20 +338,29 @@ static unsigned nbh_download_range(nbhip_state* st, int off, int cnt, double* po
     NBH_CHECK(hipSetDevice(st->device));
     const size_t n = (size_t) cnt;
     if (n == 0) return NBHIP_SUCCESS;
-    std::vector<double> tmp(n);
     double* outs[3] = { pos, vel, acc };
-    double* srcs[3][3] = { { st->px, st->py, st->pz },
-                           { st->vx, st->vy, st->vz },
-                           { st->ax, st->ay, st->az } };
+    if (st->h_bodies) {
+        double* h[3];
+        for (int o = 0; o < 3; ++o) h[o] = outs[o] ? st->h_bodies + 3 * n * o : nullptr;
+        nbh_pack_bodies(st, off, cnt, h[0], h[1], h[2]);
+        NBH_CHECK(hipGetLastError());
+        NBH_CHECK(hipStreamSynchronize(st->stream));
+        for (int o = 0; o < 3; ++o)
+            if (outs[o]) memcpy(outs[o], h[o], 3 * n * sizeof(double));
+        return NBHIP_SUCCESS;
+    }
+    double* triples = reinterpret_cast<double*>(st->su);
+    const double* srcs[3][3] = { { st->px, st->py, st->pz },
+                                 { st->vx, st->vy, st->vz },
+                                 { st->ax, st->ay, st->az } };
     for (int o = 0; o < 3; ++o) {
         if (!outs[o]) continue;
-        for (int d = 0; d < 3; ++d) {
-            NBH_CHECK(hipMemcpyAsync(tmp.data(), srcs[o][d] + off, n * sizeof(double),
-                                     hipMemcpyDeviceToHost, st->stream));
-            NBH_CHECK(hipStreamSynchronize(st->stream));
-            for (size_t i = 0; i < n; ++i) outs[o][3 * i + d] = tmp[i];
-        }
+        nbh_pack3(st->stream, cnt, srcs[o][0] + off, srcs[o][1] + off, srcs[o][2] + off, triples);
+        NBH_CHECK(hipGetLastError());
+        NBH_CHECK(hipMemcpyAsync(outs[o], triples, 3 * n * sizeof(double), hipMemcpyDeviceToHost,
+                                 st->stream));
     }
+    NBH_CHECK(hipStreamSynchronize(st->stream));
     return NBHIP_SUCCESS;
 }
 
@@ -389,12 +409,11 @@ extern "C" unsigned nbhip_batch_download(nbhip_state* st, int sim, double* pos, 
  * nbody/src/nbody_grav.c:295-303). */
 static unsigned nbh_collect(nbhip_state* st)
 {
-    DevScalars s;
-    std::vector<SimTab> tab(st->nsim);
-    NBH_CHECK(hipMemcpyAsync(&s, st->scal, sizeof(s), hipMemcpyDeviceToHost, st->stream));
-    NBH_CHECK(hipMemcpyAsync(tab.data(), st->sims, st->nsim * sizeof(SimTab),
-                             hipMemcpyDeviceToHost, st->stream));
+    nbh_export_status(st);
+    NBH_CHECK(hipGetLastError());
     NBH_CHECK(hipStreamSynchronize(st->stream));
+    const DevScalars& s = *st->h_scal;
+    const SimTab* tab = st->h_sims;
     /* st->status keeps what concerns the whole state (node capacity, launch
      * errors); h_sim_status[k] what one simulation's tree or walk reported. */
     st->status |= s.status;

@@ -605,7 +605,7 @@ extern "C" unsigned nbhip_mixed_dwarf(const nbhip_dwarf_params* p, int device, d
     const size_t n = m.nbody;
     if (n == 0) return NBHIP_SUCCESS;
     double* d = nullptr;
-    NBH_CHECK(hipMalloc((void**) &d, 7 * n * sizeof(double)));
+    NBH_CHECK(hipMalloc((void**) &d, 13 * n * sizeof(double)));
     hipStream_t s;
     hipError_t e = hipStreamCreate(&s);
     if (e != hipSuccess) {
@@ -613,10 +613,18 @@ extern "C" unsigned nbhip_mixed_dwarf(const nbhip_dwarf_params* p, int device, d
         NBH_CHECK(e);
     }
     rc = nbh_dwarf_device(p, m, d, d + n, d + 2 * n, d + 3 * n, d + 4 * n, d + 5 * n, d + 6 * n, s);
-    std::vector<double> h;
     if (!rc) {
-        h.resize(7 * n);
-        e = hipMemcpyAsync(h.data(), d, 7 * n * sizeof(double), hipMemcpyDeviceToHost, s);
+        double* triples = d + 7 * n;
+        nbh_pack3(s, (int) n, d, d + n, d + 2 * n, triples);
+        nbh_pack3(s, (int) n, d + 3 * n, d + 4 * n, d + 5 * n, triples + 3 * n);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(pos, triples, 3 * n * sizeof(double), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(vel, triples + 3 * n, 3 * n * sizeof(double),
+                               hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(mass, d + 6 * n, n * sizeof(double), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) {
             nbh_set_error("nbhip_mixed_dwarf: %s", hipGetErrorString(e));
@@ -625,15 +633,7 @@ extern "C" unsigned nbhip_mixed_dwarf(const nbhip_dwarf_params* p, int device, d
     }
     (void) hipStreamDestroy(s);
     (void) hipFree(d);
-    if (rc) return rc;
-    for (size_t i = 0; i < n; ++i) {
-        for (int k = 0; k < 3; ++k) {
-            pos[3 * i + k] = h[k * n + i];
-            vel[3 * i + k] = h[(3 + k) * n + i];
-        }
-        mass[i] = h[6 * n + i];
-    }
-    return NBHIP_SUCCESS;
+    return rc;
 }
 
 extern "C" unsigned nbhip_mixed_dwarf_state(nbhip_state* st, int sim, const nbhip_dwarf_params* p,

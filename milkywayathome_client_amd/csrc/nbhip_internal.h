@@ -166,6 +166,13 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
  * consecutive XCDs instead of one stretch of bodies an XCD: 810. */
 #define NBH_PIECES 16
 #define NBH_PIECE_BODIES (1 << 18)
+/* Bodies of at most NBH_PINNED_BODIES leave the device through the state's
+ * page-locked block, written by the packing kernel itself: with the status
+ * read the same way, an eager step of 1021 bodies and its read-back take 233
+ * us against 450 with nine copies and waits and strided loops of the host.
+ * More bodies are packed in device scratch and copied an array at a time
+ * (4 steps of 10^6 bodies and the read-back 53.0 ms against 57). */
+#define NBH_PINNED_BODIES 4096
 #define NBH_SORT_TILE 2048   /* keys per radix-sort block: 256 threads x 8 */
 #define NBH_SCAN_TILE 4096   /* items per scan block: 1024 threads x 4 */
 
@@ -263,6 +270,11 @@ struct nbhip_state {
 
     int h_level_count[64];        /* cells per level of the last eager build */
     int h_levels_valid;
+    char *h_pinned;               /* page-locked: 64 level counts, scalars, SimTab rows, and the
+                                     bodies of a state of at most NBH_PINNED_BODIES */
+    struct DevScalars *h_scal;    /* within it */
+    SimTab *h_sims;
+    double *h_bodies;
     int *h_counts_pinned;         /* pinned landing buffer of the level-count readback */
     hipEvent_t ev_counts;         /* recorded after that readback */
 
@@ -288,6 +300,13 @@ void nbh_bbox(nbhip_state* st, int drift);
 void nbh_build(nbhip_state* st, int graph_safe);
 unsigned nbh_level_lists(nbhip_state* st);
 void nbh_step_end(nbhip_state* st);
+/* x, y, z of n bodies <-> n triples (asynchronous); raw copies of device
+ * data by a kernel, which may write page-locked memory */
+void nbh_pack3(hipStream_t s, int n, const double* x, const double* y, const double* z,
+               double* out);
+void nbh_unpack3(hipStream_t s, int n, const double* in, double* x, double* y, double* z);
+void nbh_pack_bodies(nbhip_state* st, int off, int n, double* pos, double* vel, double* acc);
+void nbh_export_status(nbhip_state* st);
 void nbh_masses_changed(nbhip_state* st);
 /* launchers (walk.hip) */
 void nbh_walk(nbhip_state* st, int kick, int count, double* out_ax, double* out_ay,

@@ -1959,6 +1959,98 @@ void nbh_bbox(nbhip_state* st, int drift)
     hipLaunchKernelGGL(k_rsize, dim3(1), dim3(256), 0, st->stream, st->nsim, st->sims, st->scal);
 }
 
+/* ---------------------------------------------------------------------- */
+/* transfers                                                               */
+/* ---------------------------------------------------------------------- */
+/* The host's arrays hold triples, the device's one array a coordinate; the
+ * change of layout is the device's (a million bodies: 24 MB at memory speed),
+ * not a strided loop of the host over a copy of every array. */
+__global__ __launch_bounds__(256) void k_pack3(int n, const double* __restrict__ x,
+                                               const double* __restrict__ y,
+                                               const double* __restrict__ z,
+                                               double* __restrict__ out)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    out[3 * (size_t) i + 0] = x[i];
+    out[3 * (size_t) i + 1] = y[i];
+    out[3 * (size_t) i + 2] = z[i];
+}
+
+__global__ __launch_bounds__(256) void k_unpack3(int n, const double* __restrict__ in,
+                                                 double* __restrict__ x, double* __restrict__ y,
+                                                 double* __restrict__ z)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    x[i] = in[3 * (size_t) i + 0];
+    y[i] = in[3 * (size_t) i + 1];
+    z[i] = in[3 * (size_t) i + 2];
+}
+
+/* Positions, velocities and accelerations at once (null: not wanted). */
+__global__ __launch_bounds__(256) void k_pack_bodies(int n, const double* __restrict__ px,
+                                                     const double* __restrict__ py,
+                                                     const double* __restrict__ pz,
+                                                     const double* __restrict__ vx,
+                                                     const double* __restrict__ vy,
+                                                     const double* __restrict__ vz,
+                                                     const double* __restrict__ ax,
+                                                     const double* __restrict__ ay,
+                                                     const double* __restrict__ az,
+                                                     double* __restrict__ pos,
+                                                     double* __restrict__ vel,
+                                                     double* __restrict__ acc)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= 3 * n) return;
+    const int i = e / 3, c = e - 3 * i;
+    if (pos) pos[e] = c == 0 ? px[i] : c == 1 ? py[i] : pz[i];
+    if (vel) vel[e] = c == 0 ? vx[i] : c == 1 ? vy[i] : vz[i];
+    if (acc) acc[e] = c == 0 ? ax[i] : c == 1 ? ay[i] : az[i];
+}
+
+/* Words of the scalars and of the SimTab rows. */
+__global__ __launch_bounds__(256) void k_export(const unsigned* __restrict__ a, int na,
+                                                unsigned* __restrict__ oa,
+                                                const unsigned* __restrict__ b, int nb,
+                                                unsigned* __restrict__ ob)
+{
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < na + nb; i += gridDim.x * 256) {
+        if (i < na) oa[i] = a[i];
+        else ob[i - na] = b[i - na];
+    }
+}
+
+void nbh_pack3(hipStream_t s, int n, const double* x, const double* y, const double* z,
+               double* out)
+{
+    hipLaunchKernelGGL(k_pack3, dim3(nbh_blocks(n, 256)), dim3(256), 0, s, n, x, y, z, out);
+}
+
+void nbh_unpack3(hipStream_t s, int n, const double* in, double* x, double* y, double* z)
+{
+    hipLaunchKernelGGL(k_unpack3, dim3(nbh_blocks(n, 256)), dim3(256), 0, s, n, in, x, y, z);
+}
+
+void nbh_pack_bodies(nbhip_state* st, int off, int n, double* pos, double* vel, double* acc)
+{
+    hipLaunchKernelGGL(k_pack_bodies, dim3(nbh_blocks(3 * n, 256)), dim3(256), 0, st->stream, n,
+                       st->px + off, st->py + off, st->pz + off, st->vx + off, st->vy + off,
+                       st->vz + off, st->ax + off, st->ay + off, st->az + off, pos, vel, acc);
+}
+
+void nbh_export_status(nbhip_state* st)
+{
+    static_assert(sizeof(DevScalars) % 4 == 0 && sizeof(SimTab) % 4 == 0, "whole words");
+    const int na = (int) (sizeof(DevScalars) / 4), nb = st->nsim * (int) (sizeof(SimTab) / 4);
+    hipLaunchKernelGGL(k_export, dim3(nbh_blocks(na + nb, 256)), dim3(256), 0, st->stream,
+                       reinterpret_cast<const unsigned*>(st->scal), na,
+                       reinterpret_cast<unsigned*>(st->h_scal),
+                       reinterpret_cast<const unsigned*>(st->sims), nb,
+                       reinterpret_cast<unsigned*>(st->h_sims));
+}
+
 /* New masses: no pass has looked at them yet (nbh_plain_range). */
 __global__ __launch_bounds__(256) void k_masses_changed(int nsim, SimTab* __restrict__ sims)
 {
