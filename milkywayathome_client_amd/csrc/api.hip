@@ -973,32 +973,16 @@ extern "C" unsigned nbhip_autotune(nbhip_state* st, nbhip_tune* best, nbhip_tune
  * (root sizes persist across steps, so a recomputed step needs them) */
 static hipError_t nbh_slot_save(nbhip_state* st, double* slot, SimTab* tab)
 {
-    const size_t N = (size_t) st->n;
-    double* src[9] = { st->px, st->py, st->pz, st->vx, st->vy, st->vz, st->ax, st->ay, st->az };
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 9 && e == hipSuccess && N; ++k)
-        e = hipMemcpyAsync(slot + k * N, src[k], N * sizeof(double), hipMemcpyDeviceToDevice,
-                           st->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(tab, st->sims, st->nsim * sizeof(SimTab), hipMemcpyDeviceToDevice,
-                           st->stream);
-    return e;
+    nbh_slot_copy(st, slot, tab, 9, 1);
+    return hipGetLastError();
 }
 
 static hipError_t nbh_slot_load(nbhip_state* st, const double* slot, const SimTab* tab,
                                 int positions_only)
 {
-    const size_t N = (size_t) st->n;
-    double* dst[9] = { st->px, st->py, st->pz, st->vx, st->vy, st->vz, st->ax, st->ay, st->az };
-    hipError_t e = hipSuccess;
-    const int cnt = positions_only ? 3 : 9;
-    for (int k = 0; k < cnt && e == hipSuccess && N; ++k)
-        e = hipMemcpyAsync(dst[k], slot + k * N, N * sizeof(double), hipMemcpyDeviceToDevice,
-                           st->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(st->sims, tab, st->nsim * sizeof(SimTab), hipMemcpyDeviceToDevice,
-                           st->stream);
-    return e;
+    nbh_slot_copy(st, const_cast<double*>(slot), const_cast<SimTab*>(tab),
+                  positions_only ? 3 : 9, 0);
+    return hipGetLastError();
 }
 
 /* rebuilds the tree for the positions now in px, py, pz (nothing for Exact) */

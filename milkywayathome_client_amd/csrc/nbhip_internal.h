@@ -307,6 +307,8 @@ void nbh_pack3(hipStream_t s, int n, const double* x, const double* y, const dou
 void nbh_unpack3(hipStream_t s, int n, const double* in, double* x, double* y, double* z);
 void nbh_pack_bodies(nbhip_state* st, int off, int n, double* pos, double* vel, double* acc);
 void nbh_export_status(nbhip_state* st);
+/* the first `arrays` of x y z vx vy vz ax ay az and the SimTab rows <-> a slot */
+void nbh_slot_copy(nbhip_state* st, double* slot, SimTab* tab, int arrays, int save);
 void nbh_masses_changed(nbhip_state* st);
 /* launchers (walk.hip) */
 void nbh_walk(nbhip_state* st, int kick, int count, double* out_ax, double* out_ay,
