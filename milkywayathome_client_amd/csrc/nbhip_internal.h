@@ -55,11 +55,15 @@ struct __attribute__((aligned(16))) NodeG {
 };
 
 /* Exact criterion: the sources of a simulation of n bodies are summed in
- * this many consecutive segments (one per grid row), 1 below 4096 bodies. */
+ * this many consecutive segments (one per grid row), 1 below 4096 bodies --
+ * there the sum is the reference's, bit for bit.  Enough of them that the
+ * last round of workgroups is short: 20000 bodies are 79 x 32 workgroups, 9.9
+ * a CU (9 segments: 2.8, three rounds for two and three quarters;
+ * gradient of four steps 10.98 against 10.50 ms). */
 __host__ __device__ inline int nbh_exact_segments(int n)
 {
-    const int s = n / 2048;
-    return s < 1 ? 1 : (s > 16 ? 16 : s);
+    const int s = n / 256;
+    return n < 4096 ? 1 : (s > 32 ? 32 : s);
 }
 
 /* Per-simulation device record (one per dwarf of a batch; one for a single
