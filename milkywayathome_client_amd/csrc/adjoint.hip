@@ -245,7 +245,8 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
     const double g2 = L.valid ? gaz[j] : 0.0;
     double ox = 0.0, oy = 0.0, oz = 0.0;
 
-    L.template run<QUAD>(list + (size_t) g * NBH_LIST_CAP, len, [&](const ListRec& r, int cnt) {
+    L.template run<QUAD, true>(list + (size_t) g * NBH_LIST_CAP, len,
+                               [&](const ListRec& r, int cnt) {
         const ListHit h = L.hit(r, cnt);
         const bool use = h.use & (h.nbody != L.self);
         double v[10];

@@ -160,6 +160,7 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
  * sides' times), and of at most this many with sixteen entries a batch */
 #define NBH_LIST_BODIES (1 << 17)
 #define NBH_LIST_WIDE 8192
+#define NBH_LIST_AHEAD 24576   /* and of at most this many a batch is fetched ahead */
 
 /* Mixed and coherent walks of at most NBH_PIECE_BODIES bodies are cut into
  * NBH_PIECES parts (8 and 16 parts, one wave, us per mixed walk: 2x10^4

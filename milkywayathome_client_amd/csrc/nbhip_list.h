@@ -160,8 +160,9 @@ struct ListWave {
         return h;
     }
 
-    /* Every entry of the list, in order: batch(record, live entries). */
-    template <bool QUAD, class Batch>
+    /* Every entry of the list, in order: batch(record, live entries).  AHEAD:
+     * a batch's records are fetched while the one before is evaluated. */
+    template <bool QUAD, bool AHEAD, class Batch>
     __device__ __forceinline__ void run(const int* lst, int len, Batch&& batch)
     {
         int head = 0, tail = 0, skip = 0;             /* skip: nothing before it is met by anyone */
@@ -204,11 +205,12 @@ struct ListWave {
             }
             nbh_wave_sync();
             tail += __popcll(km);
-            /* full batches, each one's records fetched while the one before
-             * is evaluated, in two sets of registers; the last fetch may be
-             * of stale entries, whose nodes exist */
             int left = (tail - head) / S;
-            if (left > 0) {
+            if (!AHEAD) {
+                for (; left > 0; --left, head += S) batch(fetch<QUAD>(head, S), S);
+            } else if (left > 0) {
+                /* two sets of registers; the last fetch may be of stale
+                 * entries, whose nodes exist */
                 ListRec ra = fetch<QUAD>(head, S);
                 for (;;) {
                     const ListRec rb = fetch<QUAD>(head + S, S);

@@ -37,7 +37,8 @@
  *
  * Measured (lists + walk against the streaming walk, BH86 theta = 0.5 with
  * quadrupoles): 1000 bodies 120 : 386 us, 4000 202 : 890, 20 000 413 : 1520,
- * 50 000 1024 : 1795, 100 000 1970 : 2445, 200 000 4200 : 3460 -- so up to
+ * 50 000 968 : 1795, 100 000 1868 : 2445; 200 000, with a batch fetched ahead,
+ * 4200 : 3460 -- so up to
  * NBH_LIST_BODIES (131 072).  At 20 000 bodies the walk is 335 us (its
  * vector instructions alone 170) and the lists 79.  Beyond, each SIMD has
  * enough streaming waves to hide their chain, and the lists' LDS traffic
@@ -280,7 +281,7 @@ __device__ __forceinline__ int nbh_term_at(int c, int t, int T, int lane)
 }
 
 #define NBH_LW 2                      /* wavefronts per workgroup of k_walk_list */
-template <int S, bool QUAD>
+template <int S, bool QUAD, bool AHEAD>
 __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restrict__ node,
                                                            const double* __restrict__ nquad,
                                                            const double4* __restrict__ spos,
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
             simid_s, sims, scal->nmassive);
     double acc = 0.0;                                 /* of body lane % B, component lane / B */
 
-    L.template run<QUAD>(list + (size_t) g * NBH_LIST_CAP, len, [&](const ListRec& r, int cnt) {
+    L.template run<QUAD, AHEAD>(list + (size_t) g * NBH_LIST_CAP, len, [&](const ListRec& r, int cnt) {
         const ListHit h = L.hit(r, cnt);
         /* unused lanes: mass 0 and no quadrupole, at a harmless distance */
         const double m = h.use ? r.zm.y : 0.0;
@@ -405,18 +406,24 @@ void nbh_walk_list(nbhip_state* st, const WalkOut& o, double* oax, double* oay, 
     const int n = st->n;
     if (n <= 0) return;
     nbh_list_build(st);
-#define NBH_WL(S, Q)                                                                           \
-    hipLaunchKernelGGL((k_walk_list<S, Q>), dim3((n + 64 * NBH_LW / S - 1) / (64 * NBH_LW / S)),    \
+#define NBH_WL(S, Q, A)                                                                        \
+    hipLaunchKernelGGL((k_walk_list<S, Q, A>), dim3((n + 64 * NBH_LW / S - 1) / (64 * NBH_LW / S)),    \
                        dim3(64 * NBH_LW), 0,                                                   \
                        s, st->node, st->nquad, st->spos, st->perm, st->simid_s, st->sims,      \
                        st->wlist, st->wlen, oax, oay, oaz, st->vx, st->vy, st->vz, st->scal, o)
     /* Four bodies a wavefront, sixteen entries a batch, while that leaves SIMDs
      * idle: 1000 bodies 120 against 151 us (lists and walk), 4000 202 against
-     * 268, 20 000 473 against 413. */
+     * 268, 20 000 473 against 413.
+     * Eight: fetching a batch ahead takes 160 registers, three waves a SIMD;
+     * with more waves than that makes room for (24 576 bodies), a fourth wave
+     * hides more than the fetch: 20 000 bodies 338 against 352 us (the walk),
+     * 40 000 684 against 650, 100 000 1878 against 1695. */
     if (n <= NBH_LIST_WIDE) {
-        if (st->ctx.use_quad) NBH_WL(16, true); else NBH_WL(16, false);
+        if (st->ctx.use_quad) NBH_WL(16, true, true); else NBH_WL(16, false, true);
+    } else if (n <= NBH_LIST_AHEAD) {
+        if (st->ctx.use_quad) NBH_WL(8, true, true); else NBH_WL(8, false, true);
     } else {
-        if (st->ctx.use_quad) NBH_WL(8, true); else NBH_WL(8, false);
+        if (st->ctx.use_quad) NBH_WL(8, true, false); else NBH_WL(8, false, false);
     }
 #undef NBH_WL
 }

@@ -38,6 +38,12 @@ def test_body_counts(n):
     _check(plummer_bodies(n, seed=n))
 
 
+@pytest.mark.parametrize("n", [24575, 24576, 24577, 24583])
+@pytest.mark.parametrize("quad", [True, False])
+def test_end_of_the_fetch_ahead(n, quad):
+    _check(plummer_bodies(n, seed=n), theta=0.8, quad=quad, incest=True)
+
+
 @pytest.mark.parametrize("n", [131071, 131072, 131073])
 def test_largest_states_with_lists(n):
     _check(plummer_bodies(n, seed=4), theta=0.8, incest=True)   # above 1/sqrt 3 bodies meet no self
