@@ -1,5 +1,5 @@
 /*
- * Tree construction on gfx950: root-size update, Morton keys, LSD radix sort,
+ * Tree construction on gfx950: root-size update, Morton keys, their sort,
  * Karras binary radix tree (as the Cartesian tree of the adjacent prefixes),
  * octree emission in pre-order and level-by-level
  * summarisation (centre of mass, critical radius, quadrupole).
@@ -214,9 +214,9 @@ __global__ __launch_bounds__(256) void k_keys(int n, KeyView v,
 /* States of up to NBH_MERGE_BODIES bodies.  24 launches of the radix sort,
  * each a few microseconds however few the bodies, are what it costs there;
  * the merges read every other run of their group a few lines at a time, which
- * grows faster than the bodies.  Keys, sort, ties and gather, radix sort and
- * merges: 108 and 14 us (10^3 bodies), 120 and 37 (2x10^4), 127 and 53 (10^5),
- * 134 and 72 (2.6x10^5), 151 and 134 (5.2x10^5), 189 and 381 (10^6, fan 16).
+ * grows faster than the bodies.  Keys and sort, radix passes and merges: 108
+ * and 14 us (10^3 bodies), 120 and 37 (2x10^4), 127 and 53 (10^5), 134 and 72
+ * (2.6x10^5), 151 and 134 (5.2x10^5), 189 and 381 (10^6, fan 16).
  * NBH_MERGE_FAN runs at once: 8 searches advance together; 6 cost a pass more
  * at 4x10^4 (49 us to 38) and 2.6x10^5 (93 to 72), 12 and 16 search more for
  * nothing at 10^5 (57 to 53), 32 at 2x10^4 (41 to 37). */
