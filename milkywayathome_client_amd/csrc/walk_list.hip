@@ -335,7 +335,6 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
                 const double qy = r.q0.y * h.dx + r.q1.y * h.dy + r.q2.x * h.dz;
                 const double qz = r.q1.x * h.dx + r.q2.x * h.dy + r.q2.y * h.dz;
                 const double dQd = qx * h.dx + qy * h.dy + qz * h.dz;
-                /* a body's quadrupole record is zero: its terms are too */
                 double d5 = nbh_dr5<PL>(h.r2, c);
                 d5 = h.use ? d5 : 0.0;
                 const double phiQ = nbh_phiq<PL>(d5, dQd, h.r2, c);
@@ -345,6 +344,15 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
                 t[6] = -d5 * qx;
                 t[7] = -d5 * qy;
                 t[8] = -d5 * qz;
+                /* A body's quadrupole record is zero, an unused lane's d5 too,
+                 * and in the plain range everything they multiply is finite.
+                 * Outside it 1 / r^5 of a close body (itself: r^2 = eps2) or
+                 * the quadrupole of a cell that this lane opens may not be. */
+                if (!PL) {
+                    const bool live = h.use & (h.nbody < 0);
+                    #pragma unroll
+                    for (int k = 3; k < 9; ++k) t[k] = live ? t[k] : 0.0;
+                }
             }
         };
         if (L.plain) eval(std::true_type()); else eval(std::false_type());
