@@ -267,7 +267,10 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
             double cd = -3.0 * r.zm.y * s5 * dg;      /* coefficient of d */
             v[3] = s3 * dg;
             if (QUAD) {
-                /* a body's quadrupole record is zero: only its c terms are not */
+                /* a body's quadrupole record is zero, but not so what it would
+                 * be multiplied by (1 / r^9 of a close pair overflows): its
+                 * factors are replaced, and its c terms below */
+                const bool cell = h.nbody < 0;
                 const double qxx = r.q0.x, qxy = r.q0.y, qxz = r.q1.x;
                 const double qyy = r.q1.y, qyz = r.q2.x, qzz = r.q2.y;
                 const double ux = qxx * dx + qxy * dy + qxz * dz;
@@ -280,12 +283,15 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
                 const double ug = ux * g0 + uy * g1 + uz * g2;
                 const double s7 = s5 * ir2;
                 const double s9 = s7 * ir2;
-                cg += 2.5 * dQd * s7;
-                cd += -17.5 * dQd * s9 * dg + 5.0 * s7 * ug;
-                const double cu = 5.0 * s7 * dg;
-                v[0] = cg * g0 + cd * dx + cu * ux - s5 * wx;
-                v[1] = cg * g1 + cd * dy + cu * uy - s5 * wy;
-                v[2] = cg * g2 + cd * dz + cu * uz - s5 * wz;
+                const double cgq = 2.5 * dQd * s7;
+                const double cdq = -17.5 * dQd * s9 * dg + 5.0 * s7 * ug;
+                cg += cell ? cgq : 0.0;
+                cd += cell ? cdq : 0.0;
+                const double cu = cell ? 5.0 * s7 * dg : 0.0;
+                const double cw = cell ? s5 : 0.0;
+                v[0] = cg * g0 + cd * dx + cu * ux - cw * wx;
+                v[1] = cg * g1 + cd * dy + cu * uy - cw * wy;
+                v[2] = cg * g2 + cd * dz + cu * uz - cw * wz;
                 const double a = 2.5 * s7 * dg;
                 v[4] = a * dx * dx - s5 * dx * g0;
                 v[5] = 2.0 * a * dx * dy - s5 * (dy * g0 + dx * g1);
