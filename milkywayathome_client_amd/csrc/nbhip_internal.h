@@ -80,7 +80,8 @@ struct SimTab {
     unsigned flags;                /* sticky NBHIP_* bits of this simulation */
     unsigned incest;               /* a body of this simulation missed itself */
     unsigned odd_mass;             /* a mass was nonzero and outside the range of the unscaled
-                                      divisions (nbh_plain_range), or none was looked at yet */
+                                      divisions (nbh_plain_range), or a position not finite, or
+                                      none was looked at yet */
     unsigned odd_seen;             /* the same, gathered by the bbox pass that is running */
 };
 

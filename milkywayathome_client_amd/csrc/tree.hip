@@ -140,12 +140,14 @@ __global__ __launch_bounds__(256) void k_rsize(int nsim, SimTab* __restrict__ si
         SimTab& t = sims[k];
         const double xm = __longlong_as_double((long long) t.xyzmax_bits);
         double r = t.rsize;
+        unsigned odd = t.odd_seen;
         if (!(xm <= DBL_MAX)) {
             t.flags |= NBHIP_ERROR;
+            odd = 1u;                  /* a body outside every root: no plain range either */
         } else {
             while (r < 2.0 * xm) r *= 2.0;
         }
-        t.odd_mass = t.odd_seen;
+        t.odd_mass = odd;
         t.odd_seen = 0u;
         t.rsize = r;
         t.key_scale = 9223372036854775808.0 / r;
