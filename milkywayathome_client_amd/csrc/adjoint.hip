@@ -252,16 +252,19 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
         double v[10];
         auto eval = [&](auto P) {
             const double dx = h.dx, dy = h.dy, dz = h.dz;
-            double s3, ir2;
-            if (decltype(P)::value) {
-                const NbhRoot c = nbh_root(h.r2);
-                ir2 = c.ir2;
-                s3 = c.ir * c.ir2;
+            /* each power a quotient, rounded as the streaming form's */
+            constexpr bool PL = decltype(P)::value;
+            NbhRoot c;
+            auto over_r2 = [&](double a) { return PL ? nbh_quot(a, h.r2, c.ir2) : a / h.r2; };
+            double rinv;
+            if (PL) {
+                c = nbh_root(h.r2);
+                rinv = nbh_recip_refine(c.r, c.ir);
             } else {
-                ir2 = 1.0 / h.r2;
-                s3 = (1.0 / sqrt(h.r2)) / h.r2;
+                rinv = 1.0 / sqrt(h.r2);
             }
-            const double s5 = s3 * ir2;
+            const double s3 = over_r2(rinv);
+            const double s5 = over_r2(s3);
             const double dg = dx * g0 + dy * g1 + dz * g2;
             double cg = r.zm.y * s3;                  /* coefficient of g */
             double cd = -3.0 * r.zm.y * s5 * dg;      /* coefficient of d */
@@ -281,8 +284,8 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
                 const double wz = qxz * g0 + qyz * g1 + qzz * g2;
                 const double dQd = ux * dx + uy * dy + uz * dz;
                 const double ug = ux * g0 + uy * g1 + uz * g2;
-                const double s7 = s5 * ir2;
-                const double s9 = s7 * ir2;
+                const double s7 = over_r2(s5);
+                const double s9 = over_r2(s7);
                 const double cgq = 2.5 * dQd * s7;
                 const double cdq = -17.5 * dQd * s9 * dg + 5.0 * s7 * ug;
                 cg += cell ? cgq : 0.0;
