@@ -149,8 +149,11 @@ struct ListWave {
         const double drSq = h.dz * h.dz + (h.dy * h.dy + h.dx * h.dx);
         /* a node passes by itself; it is met unless it lies inside one that
          * was accepted: before this batch (lp) or in it (cont) */
-        /* a body is accepted whatever its distance (even where that is no number) */
-        const bool pass = live & ((h.nbody >= 0) | (drSq >= r.rl.x));
+        /* A body's rcrit2 is 0, and it is accepted also where the distance is
+         * no number.  (A cell of such a distance is opened; it is in the list
+         * only for a body that is no number itself, and whose sum is none
+         * either way.) */
+        const bool pass = live & !(drSq < r.rl.x);
         const unsigned long long pm = __builtin_amdgcn_ballot_w64(pass);
         const unsigned mine = (unsigned) (pm >> (b * S)) << (S - slot);
         const bool here = pass & (q >= lp) & (q < end) & ((mine & r.cont) == 0u);
