@@ -62,15 +62,17 @@ __global__ __launch_bounds__(256) void k_adj_walk(const NodeW* __restrict__ node
                                                   double* __restrict__ gxz,
                                                   double* __restrict__ gnode,
                                                   const DevScalars* __restrict__ scal,
-                                                  const int* __restrict__ wlen, AdjWalk o)
+                                                  int per, int lists, AdjWalk o)
 {
-    const int s = blockIdx.x * 256 + threadIdx.x;
     if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    /* with interaction lists, only where they did not fit */
+    if (lists && !scal->list_over) return;
     const int M = scal->nmassive;
-    const bool valid = s < o.n;
+    /* `per` bodies a wave */
+    const int lane = threadIdx.x & 63;
+    const int s = ((int) blockIdx.x * 4 + (int) (threadIdx.x >> 6)) * per + lane;
+    const bool valid = lane < per && s < o.n;
     if (__ballot(valid) == 0ull) return;
-    /* with interaction lists, only the groups that have none */
-    if (wlen && wlen[__builtin_amdgcn_readfirstlane(s >> 6)] >= 0) return;
     const double4 p = valid ? spos[s] : make_double4(0.0, 0.0, 0.0, 0.0);
     const unsigned j = valid ? perm[s] : 0u;
     const double g0 = valid ? gax[j] : 0.0;
@@ -227,14 +229,16 @@ __global__ __launch_bounds__(64 * NBH_AW) void k_adj_list(const NodeW* __restric
     __shared__ int2 s_ring[NBH_AW][NBH_LIST_RING];
     __shared__ int s_next[NBH_AW][NBH_LIST_RING];
     __shared__ double s_val[NBH_AW][V * NBH_AROW];
-    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    /* list_over: the streaming form's */
+    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) | (unsigned) scal->halt |
+        scal->list_over)
+        return;
     const int w = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int first = (blockIdx.x * NBH_AW + w) * B;
     if (first >= o.n) return;
     const int g = first >> 6;
     const int len = llen[g];
-    if (len < 0) return;                              /* the streaming form's */
     double* val = s_val[w];
     ListWave<S> L;
     L.start(node, nquad, s_ring[w], s_next[w], first, o.n, o.multi, o.all_eps2_pos != 0, spos,
@@ -529,11 +533,11 @@ void nbh_adj_force(nbhip_state* st)
     o.all_eps2_pos = st->all_eps2_pos;
     o.pot = c.pot;
     const double* ga = A->g + 6 * N;
-    dim3 grid(nbh_blocks(st->n, 256)), block(256);
-    const int* wlen = nullptr;
-    if (st->wlist && st->n > 0) {
+    const int lists = st->wlist && st->n > 0;
+    const int per = lists ? nbh_stream_bodies(st->n) : 64;
+    dim3 grid(nbh_blocks(nbh_blocks(st->n, per), 4)), block(256);
+    if (lists) {
         nbh_list_build(st);
-        wlen = st->wlen;
 #define NBH_AL(Q)                                                                              \
     hipLaunchKernelGGL((k_adj_list<Q>), dim3(nbh_blocks(st->n, 8 * NBH_AW)), dim3(64 * NBH_AW), \
                        0, s, st->node, st->nquad, st->spos, st->perm, st->simid_s, st->sims,   \
@@ -545,11 +549,11 @@ void nbh_adj_force(nbhip_state* st)
     if (c.use_quad)
         hipLaunchKernelGGL(k_adj_walk<true>, grid, block, 0, s, st->node, st->nquad, st->spos,
                            st->perm, st->simid_s, st->sims, ga, ga + N, ga + 2 * N, A->g,
-                           A->g + N, A->g + 2 * N, A->gnode, st->scal, wlen, o);
+                           A->g + N, A->g + 2 * N, A->gnode, st->scal, per, lists, o);
     else
         hipLaunchKernelGGL(k_adj_walk<false>, grid, block, 0, s, st->node, st->nquad, st->spos,
                            st->perm, st->simid_s, st->sims, ga, ga + N, ga + 2 * N, A->g,
-                           A->g + N, A->g + 2 * N, A->gnode, st->scal, wlen, o);
+                           A->g + N, A->g + 2 * N, A->gnode, st->scal, per, lists, o);
     /* roots first: a cell's record is complete before it is handed down */
     if (!st->h_levels_valid && nbh_level_lists(st) != NBHIP_SUCCESS) return;
     for (int l = 0; l < 64; ++l) {

@@ -95,6 +95,8 @@ struct DevScalars {
     int sim_bits;                  /* key bits holding the simulation id */
     unsigned long long counters[5];/* body-body, body-cell, opened, wave node steps,
                                       group far-field (cell, group) pairs */
+    unsigned list_over;            /* a group's interaction list of this tree did not fit: the
+                                      whole state streams */
     int halt;                      /* a step ended with a fatal status: later steps do nothing */
     unsigned steps_done;           /* KDK steps completed on the device */
     int level_count[64];           /* cells per level */
@@ -162,6 +164,21 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
 #define NBH_LIST_BODIES (1 << 17)
 #define NBH_LIST_WIDE 8192
 #define NBH_LIST_AHEAD 24576   /* and of at most this many a batch is fetched ahead */
+
+/* Where the lists of a state do not fit, it streams, and what bounds that is
+ * the wave with the longest chain of nodes.  Fewer bodies a wave meet fewer
+ * nodes, and up to a wave a SIMD it costs nothing: 8, 16, 32 or 64 bodies, the
+ * fewest that leave at most NBH_STREAM_WAVES waves.  A force at theta 0.2 with
+ * 512, 1024 and 2048 of them and with 64 bodies a wave, us: 9000 bodies 3019,
+ * 2948, 3114, 3618; 20000 5150, 4912, 5972, 5934; 50000 8173, 8168, 10806,
+ * 9510. */
+#define NBH_STREAM_WAVES 1024
+inline int nbh_stream_bodies(int n)
+{
+    int per = 8;
+    while (per < 64 && n > per * NBH_STREAM_WAVES) per *= 2;
+    return per;
+}
 
 /* Mixed and coherent walks of at most NBH_PIECE_BODIES bodies are cut into
  * NBH_PIECES parts (8 and 16 parts, one wave, us per mixed walk: 2x10^4

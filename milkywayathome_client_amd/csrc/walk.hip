@@ -65,15 +65,17 @@ __global__ __launch_bounds__(BS) void k_walk64(const NodeW* __restrict__ node,
                                                double* __restrict__ vy,
                                                double* __restrict__ vz,
                                                DevScalars* __restrict__ scal,
-                                               const int* __restrict__ wlen, WalkOut o)
+                                               int per, int lists, WalkOut o)
 {
-    const int s = blockIdx.x * BS + threadIdx.x;
     if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    /* with interaction lists, only where they did not fit */
+    if (lists && !scal->list_over) return;
     const int M = scal->nmassive;
-    const bool valid = s < o.n;
+    /* `per` bodies a wave */
+    const int lane = threadIdx.x & 63;
+    const int s = ((int) blockIdx.x * (BS / 64) + (int) (threadIdx.x >> 6)) * per + lane;
+    const bool valid = lane < per && s < o.n;
     if (__ballot(valid) == 0ull) return;
-    /* with interaction lists, only the groups that have none */
-    if (wlen && wlen[__builtin_amdgcn_readfirstlane(s >> 6)] >= 0) return;
     const double4 p = valid ? spos[s] : make_double4(0.0, 0.0, 0.0, 0.0);
     const LaneStart L = nbh_lane_start(s, valid, M, simid_s, sims);
     const int self = L.self, my_end = L.end;
@@ -540,17 +542,16 @@ void nbh_walk(nbhip_state* st, int kick, int count, double* oax, double* oay, do
                                st->vx, st->vy, st->vz, st->scal, o);
         return;
     }
-    /* small states: interaction lists, then the streaming walk for the groups
-     * without one (a counting walk streams them all) */
-    const int* wlen = nullptr;
-    if (st->wlist && !count) {
-        nbh_walk_list(st, o, oax, oay, oaz);
-        wlen = st->wlen;
-    }
+    /* small states: interaction lists, and the streaming walk where they do
+     * not fit (a counting walk streams) */
+    const int lists = st->wlist && !count;
+    const int per = lists ? nbh_stream_bodies(st->n) : 64;
+    grid = dim3(nbh_blocks(nbh_blocks(st->n, per), bs / 64));
+    if (lists) nbh_walk_list(st, o, oax, oay, oaz);
 #define NBH_W64(B, Q, C)                                                                     \
     hipLaunchKernelGGL((k_walk64<B, Q, C>), grid, block, 0, s, st->node, st->nquad, st->spos, \
                        st->perm, st->simid_s, st->sims, oax, oay, oaz, st->vx, st->vy, st->vz, \
-                       st->scal, wlen, o)
+                       st->scal, per, lists, o)
 #define NBH_W64B(B)                                                                          \
     if (c.use_quad) { if (count) NBH_W64(B, true, true); else NBH_W64(B, true, false); }     \
     else { if (count) NBH_W64(B, false, true); else NBH_W64(B, false, false); }

@@ -32,8 +32,8 @@
  * component) adds them entry by entry, the reference's three additions each;
  * a lane that does not interact leaves zeros, which change no bit of the sum.
  *
- * A group whose nodes do not fit the list (NBH_LIST_CAP) is left to the
- * streaming walk, which runs after this one over such groups only.
+ * Where a group's nodes do not fit its list (NBH_LIST_CAP) the whole state is
+ * left to the streaming walk, which runs after this one.
  *
  * Measured (lists + walk against the streaming walk, BH86 theta = 0.5 with
  * quadrupoles): 1000 bodies 120 : 386 us, 4000 202 : 890, 20 000 413 : 1520,
@@ -91,7 +91,7 @@ __device__ __forceinline__ ListBox nbh_list_box(bool valid, const double4& p)
 }
 
 /* Interaction list of each 64-body group: list[g * NBH_LIST_CAP ..), length
- * llen[g], -1 where it does not fit.  All waves hold the group's bodies
+ * llen[g]; scal->list_over where one does not fit.  All waves hold the group's bodies
  * (lane = body) for the box and share the nodes of a level. */
 #define NBH_LB 512                    /* threads of k_list_build */
 __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__ node,
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__
                                                     const int* __restrict__ kid,
                                                     int* __restrict__ list,
                                                     int* __restrict__ llen,
-                                                    const DevScalars* __restrict__ scal, int n,
+                                                    DevScalars* __restrict__ scal, int n,
                                                     int multi)
 {
     __shared__ unsigned s_q[NBH_LIST_CAP];            /* entry: flags and pre-order index */
@@ -124,9 +124,10 @@ __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__
     if (tid < 64) s_body[tid] = p;
     if (tid == 0) {
         s_cnt = 0;
-        s_over = 0;
+        s_over = (int) scal->list_over;               /* set meanwhile or not: one look for all */
     }
     __syncthreads();
+    if (s_over) return;                               /* another group's did not fit */
     /* the roots of the group's simulations, in pre-order */
     if (!multi) {
         if (tid == 0 && sims[0].root >= 0) {
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__
         }
         __syncthreads();
         if (s_over) {
-            if (tid == 0) llen[g] = -1;
+            if (tid == 0) scal->list_over = 1u;
             return;
         }
         lo = hi;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(NBH_LB) void k_list_build(const NodeW* __restrict__
         __syncthreads();
     }
     if (lo < hi) {                    /* deeper than 63 levels: not a tree of ours */
-        if (tid == 0) llen[g] = -1;
+        if (tid == 0) scal->list_over = 1u;
         return;
     }
     if (tid == 0) s_lev[depth] = hi;
@@ -304,14 +305,16 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
     __shared__ int2 s_ring[NBH_LW][NBH_LIST_RING];
     __shared__ int s_next[NBH_LW][NBH_LIST_RING];
     __shared__ __align__(16) double s_term[NBH_LW][3 * T * NBH_TERM_ROW];
-    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) || scal->halt) return;
+    /* list_over: the streaming walk's */
+    if ((scal->status & (NBHIP_CELL_OVERFLOW_ERROR | NBHIP_ERROR)) | (unsigned) scal->halt |
+        scal->list_over)
+        return;
     const int w = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int first = (blockIdx.x * NBH_LW + w) * B;  /* the wave's first body */
     if (first >= o.n) return;
     const int g = first >> 6;
     const int len = llen[g];
-    if (len < 0) return;                              /* the streaming walk's */
     double* term = s_term[w];
     ListWave<S> L;
     L.start(node, nquad, s_ring[w], s_next[w], first, o.n, o.multi, o.all_eps2_pos != 0, spos,
