@@ -321,7 +321,9 @@ typedef struct nbhip_tune {
 
 /* Times every setting on the current tree (call after nbhip_gravity), keeps
  * the fastest for later steps and reports it in *best; trials (may be NULL)
- * receives up to max_trials measured settings, *ntrials their count. */
+ * receives up to max_trials measured settings, *ntrials their count.  An FP64
+ * state that walks interaction lists keeps the setting it has: none shapes
+ * that walk. */
 unsigned nbhip_autotune(nbhip_state* st, nbhip_tune* best, nbhip_tune* trials, int max_trials,
                         int* ntrials);
 unsigned nbhip_set_tune(nbhip_state* st, const nbhip_tune* tune);

@@ -922,6 +922,7 @@ extern "C" unsigned nbhip_autotune(nbhip_state* st, nbhip_tune* best, nbhip_tune
     const bool mixed = st->ctx.precision != NBHIP_PRECISION_FP64;
     const int nb = group ? 3 : (mixed ? 4 : 1);
     nbhip_tune bestt = { st->tune.block, st->tune.batch, 1e300 };
+    nbhip_tune present = bestt;
     int cnt = 0;
     hipError_t e = hipSuccess;
     for (int bi = 0; bi < 3 && e == hipSuccess; ++bi) {
@@ -940,6 +941,7 @@ extern "C" unsigned nbhip_autotune(nbhip_state* st, nbhip_tune* best, nbhip_tune
             if (e != hipSuccess) break;
             float lo = fminf(ms[0], fminf(ms[1], ms[2])), hi = fmaxf(ms[0], fmaxf(ms[1], ms[2]));
             const double med = (double) (ms[0] + ms[1] + ms[2] - lo - hi);
+            if (w.block == st->tune.block && w.batch == st->tune.batch) present.ms = med;
             if (trials && cnt < max_trials) {
                 trials[cnt].block = w.block;
                 trials[cnt].batch = w.batch;
@@ -954,13 +956,19 @@ extern "C" unsigned nbhip_autotune(nbhip_state* st, nbhip_tune* best, nbhip_tune
         }
     }
     (void) hipFree(t);
+    /* interaction lists that fit: no setting shapes that walk, and the trials
+     * differ by noise alone */
+    unsigned over = 1;
+    if (e == hipSuccess && st->wlist)
+        e = hipMemcpy(&over, &st->scal->list_over, sizeof(over), hipMemcpyDeviceToHost);
     if (e != hipSuccess) {
         nbh_set_error("autotune failed: %s", hipGetErrorString(e));
         return NBHIP_GPU_ERROR;
     }
+    if (!over && present.ms < 1e300) bestt = present;
+    if (bestt.block != st->tune.block || bestt.batch != st->tune.batch) st->graph_ready = 0;
     st->tune.block = bestt.block;
     st->tune.batch = bestt.batch;
-    st->graph_ready = 0;
     if (best) *best = bestt;
     if (ntrials) *ntrials = cnt;
     return NBHIP_SUCCESS;
