@@ -169,9 +169,9 @@ __host__ __device__ inline size_t nbh_dadj_cap(int n)
  * the wave with the longest chain of nodes.  Fewer bodies a wave meet fewer
  * nodes, and up to a wave a SIMD it costs nothing: 8, 16, 32 or 64 bodies, the
  * fewest that leave at most NBH_STREAM_WAVES waves.  A force at theta 0.2 with
- * 512, 1024 and 2048 of them and with 64 bodies a wave, us: 9000 bodies 3019,
- * 2948, 3114, 3618; 20000 5150, 4912, 5972, 5934; 50000 8173, 8168, 10806,
- * 9510. */
+ * 512, 1024 and 2048 of them, and from the streaming walk alone with 64 bodies
+ * a wave, us: 9000 bodies 3019, 2948, 3114, 3618; 20000 5150, 4912, 5972,
+ * 5934; 50000 8173, 8168, 10806, 9510. */
 #define NBH_STREAM_WAVES 1024
 inline int nbh_stream_bodies(int n)
 {
@@ -269,7 +269,7 @@ struct nbhip_state {
     int *blist;                   /* summaries: inside cells of each body block, by level */
     int *span, *span_sorted;      /* summaries: cells spanning body blocks / super-blocks */
     int *wlist, *wlen;            /* FP64 list walk: each 64-body group's nodes in pre-order
-                                     (NBH_LIST_CAP slots) and their count, -1: streaming walk */
+                                     (NBH_LIST_CAP slots) and their count */
     double *wsum;                 /* mixed walk in parts: each part's sums and their errors */
     unsigned *wmet;               /* and 0 where a body met its own record */
     double *exact_part;           /* Exact criterion: per-segment partial sums */

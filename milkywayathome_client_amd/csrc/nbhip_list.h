@@ -118,7 +118,8 @@ struct ListWave {
         const int2 e = ring[(head + slot) & (NBH_LIST_RING - 1)];
         r.q = slot < cnt ? (unsigned) e.x : 0u;
         r.cont = (unsigned) e.y;
-        /* 32-bit offsets: a state with lists has under 2^21 nodes */
+        /* 32-bit offsets: a body is the first of at most 64 cells, one a level */
+        static_assert(65ull * NBH_LIST_BODIES * 48 < 1ull << 32, "node offsets");
         const unsigned off = r.q * 48u;
         const double2* rec =
             reinterpret_cast<const double2*>(reinterpret_cast<const char*>(node) + off);

@@ -787,7 +787,7 @@ __global__ __launch_bounds__(1024) void k_nscan_part(unsigned* __restrict__ part
  * cell and node counts and the flag of a table overflow from the last massive
  * body -- with one simulation also its end and depth (k_sim_ends otherwise).
  * The last workgroup builds the min-hierarchy's levels from 3 up.  One launch
- * of 5 us (2x10^4 bodies) instead of six of 2.3 to 4.4, 14 at 10^6. */
+ * of 5 us (2x10^4 bodies) instead of six of 2.3 to 4.4, 8 at 10^5, 14 at 10^6. */
 __global__ __launch_bounds__(256) void k_cells(int n, const int* __restrict__ simid_s,
                                                unsigned* __restrict__ cincl,
                                                const unsigned* __restrict__ part, int node_cap,

@@ -384,8 +384,9 @@ __global__ __launch_bounds__(BS) void k_walk32(const NodeF* __restrict__ node,
     nbh_walk_finish(o, p.x, p.y, p.z, ax, ay, az, perm[s], oax, oay, oaz, vx, vy, vz);
 }
 
-/* The parts of a split mixed walk added up, and the step finished: 816 bytes
- * read per body, consecutive lanes consecutive addresses. */
+/* The parts of a split mixed walk added up, and the step finished: 868 bytes
+ * read per body (16 parts of 52, position and index), consecutive lanes
+ * consecutive addresses. */
 __global__ __launch_bounds__(256) void k_walk_fold(const double* __restrict__ wsum,
                                                    const unsigned* __restrict__ wmet,
                                                    const double4* __restrict__ spos,
