@@ -676,6 +676,13 @@ static unsigned nbh_tree_segment(nbhip_state* st, int first, int nn, int body_of
     if (st->n > 0)
         NBH_CHECK(hipMemcpy(perm.data(), st->perm, st->n * sizeof(unsigned),
                             hipMemcpyDeviceToHost));
+    /* a build that met an inconsistency leaves records unwritten */
+    for (int i = 0; i < nn; ++i)
+        if (nodes[i].body >= st->n) {
+            nbh_set_error("incomplete tree: node %d of %d names body %d of %d", i, nn,
+                          nodes[i].body, st->n);
+            return NBHIP_ERROR;
+        }
     for (int i = 0; i < nn; ++i) {
         const NodeW& w = nodes[i];
         const bool body = w.body >= 0;
