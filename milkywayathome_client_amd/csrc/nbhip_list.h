@@ -73,6 +73,7 @@ struct ListWave {
     bool valid, plain, eps2_pos, met;
     double4 p;
     double eps2;
+    int spare;                       /* an entry of the list: the node of lanes without one */
     int lp, end, self;               /* place in the body's walk, its simulation's end */
     double bx[B], by[B], bz[B];      /* the wave's bodies, uniform (past the last: the first) */
 
@@ -104,7 +105,13 @@ struct ListWave {
         end = multi ? st.end : INT_MAX;
         self = valid && body < nmassive ? body : -2;
         eps2_pos = eps2_pos_;
-        plain = __builtin_amdgcn_ballot_w64(!nbh_plain_range(st)) == 0ull;
+        /* plain: every simulation of the group, whose nodes are in the list */
+        bool odd = !nbh_plain_range(st);
+        if (multi) {
+            const int o = (first & ~63) + lane;
+            odd = !nbh_plain_range(sims[simid_s[o < n ? o : first]]);
+        }
+        plain = __builtin_amdgcn_ballot_w64(odd) == 0ull;
         met = false;
         rnext[lane] = rnext[lane + 64] = 0;
         ring[lane] = ring[lane + 64] = make_int2(0, 0);
@@ -116,7 +123,7 @@ struct ListWave {
     {
         ListRec r;
         const int2 e = ring[(head + slot) & (NBH_LIST_RING - 1)];
-        r.q = slot < cnt ? (unsigned) e.x : 0u;
+        r.q = (unsigned) (slot < cnt ? e.x : spare);
         r.cont = (unsigned) e.y;
         /* 32-bit offsets: a body is the first of at most 64 cells, one a level */
         static_assert(65ull * NBH_LIST_BODIES * 48 < 1ull << 32, "node offsets");
@@ -175,6 +182,7 @@ struct ListWave {
         int q_next = lane < len ? lst[lane] : 0;
         NodeW nd_next = node[q_next];
         int q_after = 64 + lane < len ? lst[64 + lane] : 0;
+        spare = __builtin_amdgcn_readfirstlane(q_next);
         nbh_wave_sync();
         for (int i0 = 0; i0 < len; i0 += 64) {
             const bool in = i0 + lane < len;

@@ -347,15 +347,16 @@ __global__ __launch_bounds__(64 * NBH_LW) void k_walk_list(const NodeW* __restri
                 t[6] = -d5 * qx;
                 t[7] = -d5 * qy;
                 t[8] = -d5 * qz;
-                /* A body's quadrupole record is zero, an unused lane's d5 too,
-                 * and in the plain range everything they multiply is finite.
-                 * Outside it 1 / r^5 of a close body (itself: r^2 = eps2) or
-                 * the quadrupole of a cell that this lane opens may not be. */
-                if (!PL) {
-                    const bool live = h.use & (h.nbody < 0);
-                    #pragma unroll
-                    for (int k = 3; k < 9; ++k) t[k] = live ? t[k] : 0.0;
-                }
+            }
+            /* A body's quadrupole record is zero, an unused lane's mass and d5
+             * too, and in the plain range everything they multiply is finite.
+             * Outside it 1 / r^5 of a close body (itself: r^2 = eps2), the
+             * quadrupole of a cell that this lane opens or the place of another
+             * simulation's node may not be. */
+            if (!PL) {
+                #pragma unroll
+                for (int k = 0; k < 3 * T; ++k)
+                    t[k] = h.use & (k < 3 || h.nbody < 0) ? t[k] : 0.0;
             }
         };
         if (L.plain) eval(std::true_type()); else eval(std::false_type());
